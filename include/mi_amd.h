@@ -197,6 +197,11 @@ int mi_decode_static(const void* q, int64_t q_stride_batch, int64_t q_stride_hea
  * plan() takes the head counts and head_dim (as FlashInfer's plan does): a
  * workgroup serves all num_qo_heads / num_kv_heads (1..8) Q heads of one KV
  * head, and the query positions per workgroup depend on both.
+ * A workspace larger than mi_prefill_workspace_size also holds partial
+ * results at its end (never more than three quarters of it): launches of few
+ * rows over many keys are then cut along the keys and merged.  128 MiB is
+ * enough for every shape; a smaller one only splits less, with the same
+ * results within rounding.
  * head_dim in {64, 128, 256}; page_size == 16.
  * ------------------------------------------------------------------------ */
 size_t mi_prefill_workspace_size(int32_t batch_size, int64_t total_q);

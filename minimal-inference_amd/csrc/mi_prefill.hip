@@ -14,10 +14,13 @@
 // for group 4), so every K/V byte the workgroup stages serves all the heads
 // of its group.  (8-wave workgroups over twice the positions halve the
 // staging per wave but measured 10 % slower: two independent 4-wave
-// workgroups per CU keep computing across each other's barriers.)  plan()
-// lists the tiles request
+// workgroups per CU keep computing across each other's barriers.)  Launches
+// that leave most of the chip idle take fine tiles of one row block per wave
+// instead, and tiles with long key ranges are cut into units along the keys
+// whose fp32 partials the last unit merges (prefill_plan_kernel says when and
+// why).  plan() lists the units request
 // by request (longest prompt first), each request's tiles heaviest first; the
-// grid maps tile-major, so the XCD that a KV head's workgroups land on runs
+// grid maps unit-major, so the XCD that a KV head's workgroups land on runs
 // one request's tiles back to back and finds its K / V in L2.
 //
 // Per 64-key tile: the workgroup stages K and V in LDS (double buffered: the
@@ -35,6 +38,7 @@
 //                   transpose read in the same key order.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "mi_common.h"
@@ -50,9 +54,6 @@ constexpr int kPageSize = 16;
 constexpr int kMinRows = 8;    // fewest query positions per workgroup (head_dim 256, group 8)
 constexpr int kKvTile = 64;    // keys per staged tile (4 pages)
 constexpr float kLazyRescale = 8.0f;
-#ifndef PREFILL_WAVES
-#define PREFILL_WAVES 2
-#endif
 // 32-byte row pad: the transpose reads of V (four rows x 32 bytes per
 // 16 lanes) and the 16-byte K reads both land on distinct banks (a 16-byte
 // pad measured 13.9M bank-conflict cycles per launch on the Mistral-7B
@@ -73,43 +74,104 @@ constexpr float kLazyRescale = 8.0f;
 // transpose reads of two lane groups fall on distinct banks.
 constexpr int kOutPad = 144;
 
+// One work unit of the run: the KV tiles [kt_begin, kt_end) of one query tile.
+// A query tile whose keys are cut into `nsplit` > 1 units has consecutive
+// units, each with its own partial slot.
 struct alignas(32) PrefillTile {
-  int b;
   int q_begin;  // absolute first query row of the tile
   int q_rows;   // positions in this tile (<= bm)
   int qo_len;
   int kv_len;
   int row0;           // first position of the tile within its request
   int kv_page_begin;  // absolute position of the request's first page in kv_indices
-  int pad;
+  int kt;             // kt_begin | kt_end << 16 (kToEnd: to the tile's last key)
+  int part;           // partial slot << 16 | split << 8 | nsplit (nsplit <= 1: the whole tile)
 };
+constexpr unsigned kToEnd = 0xffffu;
 
 struct PrefillHeader {
   int num_tiles;
   int error;
-  int bm;
-  int pad;
+  int bm;             // query positions per tile
+  int row_blocks;     // 16-row blocks per wave: the coarse or the fine form of the tiles
+  int chunk;          // KV tiles per unit at most (0: no tile is split)
+  int slots;          // partial slots per KV head (the counters follow them)
+  int64_t split_off;  // byte offset of the partial slots in the workspace
 };
 
 // Waves per workgroup.
 constexpr int waves_for(int /*head_dim*/) { return 4; }
 
-// Row blocks of 16 (position, head) rows per wave: three for head_dim 128
-// (each K / V operand read from LDS then feeds three blocks), two for 64, one
-// for 256.
-int row_blocks(int /*group*/, int head_dim) { return head_dim > 128 ? 1 : head_dim == 128 ? 3 : 2; }
+// Row blocks of 16 (position, head) rows per wave of the coarse tiles: three
+// for head_dim 128 (each K / V operand read from LDS then feeds three blocks),
+// two for 64, one for 256.  The fine tiles have one.
+constexpr int row_blocks(int head_dim) { return head_dim > 128 ? 1 : head_dim == 128 ? 3 : 2; }
 
 // Query positions per workgroup: the workgroup's 16 * waves * row blocks rows
 // hold bm positions x group heads, bm = rows / group.
-int rows_per_tile(int group, int head_dim) {
-  const int bm = 16 * waves_for(head_dim) * row_blocks(group, head_dim) / group;
-  return bm < kMinRows ? kMinRows : bm;
-}
+int rows_per_tile(int group, int head_dim, int blocks) { return 16 * waves_for(head_dim) * blocks / group; }
 
 size_t tile_capacity(int batch, int64_t total_q) { return size_t(total_q / kMinRows + batch + 1); }
 
 size_t prefill_ws_bytes(int batch, int64_t total_q) {
   return 256 + mi::align_up(tile_capacity(batch, total_q) * sizeof(PrefillTile), 256);
+}
+
+// Workgroups resident at once: two per CU at head_dim 128 (registers), three
+// at 64, one at 256 (LDS).
+int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 3 : head_dim == 128 ? 2 : 1); }
+
+// Fine tiles are for launches that leave most of the chip idle: a KV tile
+// takes a workgroup of one row block per wave 1.1-1.3 us instead of the 2.2-2.8
+// us of three, so a chain of them is half as long and a merge moves a third of
+// the bytes, but the K / V operands read from LDS feed a third of the MFMAs.
+// Measured on Mistral-7B heads, whole coarse tiles / coarse and split / fine
+// (and split): one prompt of 512 tokens 23.9 / 21.8 / 13.5 us, 1,024: 41.0 /
+// 36.2 / 25.3, 64 new tokens on 8,000 cached 267 / 66.5 / 31.7; 2,048: 79 / 54 /
+// 60; four turns of 61-413 tokens on 2,000-6,000 cached 199 / 89 / 132;
+// Qwen2.5-7B heads, one prompt of 1,537: 59 / 41 / 44.  So: fine while the load per resident workgroup, counted in fine KV
+// tiles, is at most kFineLoad.
+constexpr int kFineLoad = 12;
+constexpr int kFineRounds = 4;  // resident rounds of fine units at most
+
+// Workgroups of the run: whole resident rounds over the most coarse tiles the
+// rows can make, or the units that a plan of fine tiles may hold.  The plan
+// never makes more.
+int64_t run_groups(int batch, int64_t total_q, int group, int hkv, int head_dim) {
+  const int64_t res = resident_groups(head_dim);
+  const auto groups = [&](int blocks) { return (total_q / rows_per_tile(group, head_dim, blocks) + batch) * hkv; };
+  const int64_t coarse = (groups(row_blocks(head_dim)) + res - 1) / res * res;
+  const int64_t fine = (groups(1) + res - 1) / res * res;
+  return std::max(coarse, std::min(fine, kFineRounds * res));
+}
+
+// A split unit's partial, per KV head: the workgroup's O accumulators in lane
+// order and (m, l) per lane and row block, all fp32.
+constexpr size_t partial_bytes(int head_dim, int blocks) {
+  return size_t(waves_for(head_dim)) * blocks * (head_dim / 16 * 1024 + 512);
+}
+constexpr int kCounterStride = 32;  // ints: one 128-byte line per merge counter
+constexpr int kMaxSplits = 64;      // per tile
+
+// Partial slots per KV head of coarse and of fine units and their offset: the
+// end of the workspace, at most three quarters of it and two resident rounds
+// of coarse units.  No slots when the workspace is too small to be worth
+// splitting for: the plan then splits nothing.
+struct PartialLayout {
+  size_t off;
+  int coarse, fine;
+};
+PartialLayout partial_layout(size_t workspace_bytes, int hkv, int head_dim) {
+  const auto per = [&](int blocks) { return (partial_bytes(head_dim, blocks) + kCounterStride * sizeof(int)) * size_t(hkv); };
+  PartialLayout L{0, 0, 0};
+  const size_t c = std::min(workspace_bytes / 4 * 3 / per(row_blocks(head_dim)),
+                            size_t(2 * resident_groups(head_dim) / hkv));
+  const size_t bytes = c * per(row_blocks(head_dim)) + 256;
+  if (c < 2 || bytes + 256 + sizeof(PrefillTile) > workspace_bytes) return L;
+  L.off = (workspace_bytes - c * per(row_blocks(head_dim))) & ~size_t(255);
+  L.coarse = int(c);
+  L.fine = int(std::min(c * per(row_blocks(head_dim)) / per(1), size_t(0xffff)));
+  return L;
 }
 
 struct PlanParams {
@@ -118,89 +180,309 @@ struct PlanParams {
   const int32_t* last_page_len;
   int batch;
   int capacity;
-  int bm;
+  int group, hkv;
+  int bm[2], blocks[2], slots[2];  // positions, row blocks per wave and partial slots of fine [0] and coarse [1] tiles
+  size_t counters_off[2];          // of the merge counters, behind the partials
+  int resident;                    // workgroups resident at once
+  int split_capacity;              // units the list holds in front of the partial slots
+  int64_t split_off;
+  char* ws;
   PrefillHeader* header;
   PrefillTile* tiles;
 };
 
-// Inclusive scan over the block; *total gets the block-wide sum.  Ends with a
-// barrier so `buf` may be reused at once.
-__device__ int block_scan(int v, int* buf, int* total) {
-  const int t = threadIdx.x;
-  buf[t] = v;
-  __syncthreads();
-  for (int o = 1; o < int(blockDim.x); o <<= 1) {
-    const int add = (t >= o) ? buf[t - o] : 0;
-    __syncthreads();
-    buf[t] += add;
-    __syncthreads();
+constexpr int kPlanThreads = 1024;
+constexpr int kSplitTiles = 8192;  // most query tiles whose keys are considered for splitting
+constexpr int kMinChunk = 4;  // KV tiles per unit at least (2 and 3 measured the same on a 512-token prompt)
+
+// Inclusive scan over the block: shuffles inside each wave, then the wave
+// totals through LDS.  *total gets the block-wide sum.
+__device__ int block_scan(int v, int* wsum, int* total) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(v, o);
+    if (lane >= o) v += y;
   }
-  const int r = buf[t];
-  *total = buf[blockDim.x - 1];
+  __syncthreads();  // the previous call's readers are done with wsum
+  if (lane == 63) wsum[w] = v;
   __syncthreads();
-  return r;
+  int pre = 0, tot = 0;
+  for (int i = 0; i < kPlanThreads / 64; ++i) {
+    const int s = wsum[i];
+    pre += (i < w) ? s : 0;
+    tot += s;
+  }
+  *total = tot;
+  return v + pre;
 }
 
-// Tile order: requests by decreasing prompt length (ties by index), each
-// request's tiles from the end of its prompt (most keys) to the start.  The
-// run kernel maps consecutive tiles of one (request, KV head) to consecutive
-// workgroups of one XCD, so they share the request's K / V in that XCD's L2.
-__global__ __launch_bounds__(1024) void prefill_plan_kernel(PlanParams p) {
-  __shared__ int buf[1024];
-  const int t = threadIdx.x;
+__device__ __forceinline__ int request_kv(const PlanParams& p, int b) {
+  const int np = max(0, p.kv_indptr[b + 1] - p.kv_indptr[b]);
+  return np > 0 ? (np - 1) * kPageSize + min(max(p.last_page_len[b], 1), kPageSize) : 0;
+}
+
+__device__ __forceinline__ PrefillTile make_tile(int bm, int qo, int kv, int q0, int pb0, int nt, int k) {
+  PrefillTile tile;
+  tile.row0 = (nt - 1 - k) * bm;
+  tile.q_begin = q0 + tile.row0;
+  tile.q_rows = min(bm, qo - tile.row0);
+  tile.qo_len = qo;
+  tile.kv_len = kv;
+  tile.kv_page_begin = pb0;
+  tile.kt = int(kToEnd << 16);
+  tile.part = 0;
+  return tile;
+}
+
+__device__ __forceinline__ void write_header(const PlanParams& p, int form, int units, int ntiles, int chunk) {
+  p.header->num_tiles = units;
+  p.header->error = ntiles > p.capacity ? 1 : 0;
+  p.header->bm = p.bm[form];
+  p.header->row_blocks = p.blocks[form];
+  p.header->chunk = chunk;
+  p.header->slots = p.slots[form];
+  p.header->split_off = p.split_off;
+}
+
+// Batches of more requests than the block has threads: one request per thread
+// and round, its place found by counting the requests ordered before it in
+// global memory; coarse tiles, none of them split.
+__device__ void plan_large(const PlanParams& p, int* wsum) {
+  const int t = threadIdx.x, bm = p.bm[1];
   int total = 0;
   for (int base = 0; base < p.batch; base += blockDim.x) {
     const int b = base + t;
     int nt = 0, start = 0;
     if (b < p.batch) {
       const int qo = max(0, p.qo_indptr[b + 1] - p.qo_indptr[b]);
-      nt = (qo + p.bm - 1) / p.bm;
-      // tiles of the requests ordered before b
+      nt = (qo + bm - 1) / bm;
       for (int c = 0; c < p.batch; ++c) {
         const int qc = max(0, p.qo_indptr[c + 1] - p.qo_indptr[c]);
-        if (qc > qo || (qc == qo && c < b)) start += (qc + p.bm - 1) / p.bm;
+        if (qc > qo || (qc == qo && c < b)) start += (qc + bm - 1) / bm;
       }
-      if (start + nt <= p.capacity) {
-        const int np = max(0, p.kv_indptr[b + 1] - p.kv_indptr[b]);
-        const int kv = np > 0 ? (np - 1) * kPageSize + min(max(p.last_page_len[b], 1), kPageSize) : 0;
-        for (int k = 0; k < nt; ++k) {
-          PrefillTile tile;
-          tile.b = b;
-          tile.row0 = (nt - 1 - k) * p.bm;
-          tile.q_begin = p.qo_indptr[b] + tile.row0;
-          tile.q_rows = min(p.bm, qo - tile.row0);
-          tile.qo_len = qo;
-          tile.kv_len = kv;
-          tile.kv_page_begin = p.kv_indptr[b];
-          tile.pad = 0;
-          p.tiles[start + k] = tile;
-        }
-      }
+      if (start + nt <= p.capacity)
+        for (int k = 0; k < nt; ++k)
+          p.tiles[start + k] = make_tile(bm, qo, request_kv(p, b), p.qo_indptr[b], p.kv_indptr[b], nt, k);
     }
     int chunk_total = 0;
-    block_scan(nt, buf, &chunk_total);
+    block_scan(nt, wsum, &chunk_total);
     total += chunk_total;
   }
-  if (t == 0) {
-    p.header->num_tiles = min(total, p.capacity);
-    p.header->error = total > p.capacity ? 1 : 0;
-    p.header->bm = p.bm;
+  if (t == 0) write_header(p, 1, min(total, p.capacity), total, 0);
+}
+
+// Tile order: requests by decreasing prompt length (ties by index), each
+// request's tiles from the end of its prompt (most keys) to the start.  The
+// run kernel maps consecutive tiles of one (request, KV head) to consecutive
+// workgroups of one XCD, so they share the request's K / V in that XCD's L2.
+//
+// Splitting.  A tile's keys are a serial chain of KV tiles that take about as
+// long whether one or two workgroups share the CU, so a launch of few tiles
+// (one prompt, a short turn on a long cached context) lasts as long as its
+// longest tile while most of the chip idles.  Tiles of more than `chunk` KV
+// tiles are therefore cut into near-equal units whose partial results the last
+// unit to finish merges.  chunk is the smallest value of at least
+//   * the load that fills every resident workgroup evenly (so launches of many
+//     rounds, whose tiles balance by themselves, split nothing),
+//   * kMinChunk, and sqrt(longest / 2): a further split costs its merger about
+//     half a KV tile,
+// whose units fit the rounds that the unsplit tiles need.  Coarse tiles split
+// only to fill one round (split over a second one, a 4,096-token prompt went
+// 160 -> 168 us: the partials of three row blocks are 104 KB per unit).  The
+// count assumes a causal run; the last
+// unit of a tile takes whatever keys remain, so a non-causal run of the same
+// plan is complete too.
+__global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p) {
+  __shared__ int s_qo[kPlanThreads], s_kv[kPlanThreads], s_q0[kPlanThreads], s_pb0[kPlanThreads];
+  __shared__ int s_req[kPlanThreads], s_end[kPlanThreads], wsum[kPlanThreads / 64];
+  __shared__ int red[2][kPlanThreads / 64], ok[2][kPlanThreads / 64], s_fit;
+  __shared__ unsigned short s_n[kSplitTiles];
+  if (p.batch > kPlanThreads) {
+    plan_large(p, wsum);
+    return;
   }
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  constexpr int NW = kPlanThreads / 64;
+  int qo = 0;
+  float area = 0.f, fine_tiles = 0.f;  // this request's (row, key) pairs with half a KV tile of masked ones per row
+  if (t < p.batch) {
+    const int q0 = p.qo_indptr[t], q1 = p.qo_indptr[t + 1], pb0 = p.kv_indptr[t], pb1 = p.kv_indptr[t + 1];
+    const int lpl = p.last_page_len[t];
+    const int np = max(0, pb1 - pb0);
+    const int kv = np > 0 ? (np - 1) * kPageSize + min(max(lpl, 1), kPageSize) : 0;
+    qo = max(0, q1 - q0);
+    s_qo[t] = qo;
+    s_q0[t] = q0;
+    s_pb0[t] = pb0;
+    s_kv[t] = kv;
+    area = float(qo) * (max(0.f, float(kv) - 0.5f * float(qo)) + 0.5f * kKvTile);
+    fine_tiles = float((qo + p.bm[0] - 1) / p.bm[0]);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    area += __shfl_xor(area, o);
+    fine_tiles += __shfl_xor(fine_tiles, o);
+  }
+  if (lane == 0) {
+    red[0][w] = __float_as_int(area);
+    red[1][w] = __float_as_int(fine_tiles);
+  }
+  if (t == 0) s_fit = 0;
+  __syncthreads();
+  area = fine_tiles = 0.f;
+  for (int i = 0; i < NW; ++i) {
+    area += __int_as_float(red[0][i]);
+    fine_tiles += __int_as_float(red[1][i]);
+  }
+  // fine or coarse tiles (see kFineLoad)
+  const float fine_load = area * float(p.group * p.hkv) / (64.f * kKvTile * float(p.resident));
+  const int form = p.blocks[1] > 1 && fine_load <= float(kFineLoad) &&
+                           fine_tiles * float(p.hkv) <= float(kFineRounds * p.resident) ? 0 : 1;
+  const int bm = p.bm[form], nslots = p.slots[form];
+  int rank = 0;
+  for (int c = 0; c < p.batch; ++c) {
+    const int qc = s_qo[c];
+    rank += (qc > qo || (qc == qo && c < t)) ? 1 : 0;
+  }
+  if (t < p.batch) {
+    s_req[rank] = t;
+    s_end[rank] = (qo + bm - 1) / bm;
+  }
+  __syncthreads();
+  int ntiles = 0;
+  const int end = block_scan(t < p.batch ? s_end[t] : 0, wsum, &ntiles);
+  s_end[t] = end;
+  if (t < p.batch && end <= p.capacity) atomicMax(&s_fit, end);
+  __syncthreads();
+  const int fit = s_fit;  // tiles of the requests that fit the list
+
+  // tile i of the list: its request's rank, and its causal KV tiles
+  auto rank_of = [&](int i) {
+    int lo = 0, hi = p.batch - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (s_end[mid] > i) hi = mid; else lo = mid + 1;
+    }
+    return lo;
+  };
+  auto tile_of = [&](int i) {
+    const int r = rank_of(i), b = s_req[r];
+    const int nt = (s_qo[b] + bm - 1) / bm;
+    return make_tile(bm, s_qo[b], s_kv[b], s_q0[b], s_pb0[b], nt, i - (s_end[r] - nt));
+  };
+  auto kv_tiles = [&](const PrefillTile& x) {
+    return (max(0, min(x.kv_len, x.row0 + x.q_rows + x.kv_len - x.qo_len)) + kKvTile - 1) / kKvTile;
+  };
+  // the units that fill the rounds which the unsplit tiles need
+  const int rounds = (ntiles * p.hkv + p.resident - 1) / p.resident;
+  const int limit = min(rounds * p.resident / p.hkv, p.split_capacity);
+  const bool consider = nslots > 0 && (form == 0 || rounds == 1) && ntiles == fit && ntiles <= min(kSplitTiles, limit);
+  int chunk = 0, longest = 0;
+  if (consider) {
+    int sum = 0;
+    for (int i = t; i < ntiles; i += kPlanThreads) {
+      const int n = kv_tiles(tile_of(i));
+      s_n[i] = (unsigned short)min(n, 65535);
+      sum += n;
+      longest = max(longest, n);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      sum += __shfl_xor(sum, o);
+      longest = max(longest, __shfl_xor(longest, o));
+    }
+    if (lane == 0) {
+      red[0][w] = sum;
+      red[1][w] = longest;
+    }
+    __syncthreads();
+    long long total = 0;
+    for (int i = 0; i < NW; ++i) {
+      total += red[0][i];
+      longest = max(longest, red[1][i]);
+    }
+    int lo = max(kMinChunk, int((total * p.hkv + p.resident - 1) / p.resident));
+    lo = max(lo, max((longest + kMaxSplits - 1) / kMaxSplits, int(sqrtf(0.5f * float(longest)))));
+    int hi = longest;
+    if (longest < int(kToEnd)) {
+      // every wave tries one value between lo and hi per round; the units and
+      // the partial slots fall as the value grows, and `longest` fits
+      for (int round = 0; lo < hi; ++round) {
+        const int c = lo + (w + 1) * (hi - lo) / (NW + 1);
+        int units = 0, parts = 0;
+        for (int i = lane; i < ntiles; i += 64) {
+          const int ns = max(1, (int(s_n[i]) + c - 1) / c);
+          units += ns;
+          parts += ns > 1 ? ns : 0;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+          units += __shfl_xor(units, o);
+          parts += __shfl_xor(parts, o);
+        }
+        if (lane == 0) ok[round & 1][w] = units <= limit && parts <= nslots;
+        __syncthreads();
+        int nlo = lo, nhi = hi;
+        for (int i = 0; i < NW; ++i) {
+          const int ci = lo + (i + 1) * (hi - lo) / (NW + 1);
+          if (ok[round & 1][i]) nhi = min(nhi, ci); else nlo = max(nlo, ci + 1);
+        }
+        lo = nlo;
+        hi = nhi;
+      }
+      chunk = lo < longest ? lo : 0;
+    }
+  }
+  int units = fit;
+  if (chunk == 0) {
+    for (int i = t; i < fit; i += kPlanThreads) p.tiles[i] = tile_of(i);
+  } else {
+    // units in tile order; the scan carries the units and, above them, the
+    // partial slots before each tile
+    units = 0;
+    int slots = 0;
+    for (int base = 0; base < ntiles; base += kPlanThreads) {
+      const int i = base + t;
+      const int n = i < ntiles ? int(s_n[i]) : 0;
+      const int ns = i < ntiles ? max(1, (n + chunk - 1) / chunk) : 0;
+      const int mine = ns | (ns > 1 ? ns << 16 : 0);
+      int all = 0;
+      const int before = block_scan(mine, wsum, &all) - mine;
+      if (i < ntiles) {
+        PrefillTile x = tile_of(i);
+        const int u0 = units + (before & 0xffff), slot0 = slots + (before >> 16);
+        for (int s = 0; s < ns; ++s) {
+          const unsigned kb = unsigned(s * n / ns), ke = s + 1 < ns ? unsigned((s + 1) * n / ns) : kToEnd;
+          x.kt = int(kb | ke << 16);
+          x.part = ns > 1 ? ((slot0 + s) << 16 | s << 8 | ns) : 0;
+          p.tiles[u0 + s] = x;
+        }
+      }
+      units += all & 0xffff;
+      slots += all >> 16;
+      __syncthreads();
+    }
+    int* counters = reinterpret_cast<int*>(p.ws + p.counters_off[form]);
+    for (int i = t; i < slots * p.hkv; i += kPlanThreads) counters[i * kCounterStride] = 0;
+  }
+  if (t == 0) write_header(p, form, units, ntiles, chunk);
 }
 
 struct RunParams {
+  char* ws;
   const PrefillHeader* header;
   const PrefillTile* tiles;
   const uint16_t* q;
   int64_t q_st, q_sh;
   int64_t q_ext;  // elements one position's heads span: (heads - 1) * q_sh + head_dim
   const uint16_t* pool;
-  int64_t num_pages;
+  unsigned num_pages;  // page ids are 32-bit: capped there
   const int32_t* indices;
   uint16_t* out;
   int64_t o_st, o_sh, o_ext;
   int64_t total_q;
-  int hkv, group, causal, bm;
+  int hkv, group, causal;
   float scale_log2;
 };
 
@@ -286,25 +568,158 @@ struct PrefillTraits {
   static constexpr int SMEM = 2 * 2 * TILE > WAVES * MAXRB * OB ? 2 * 2 * TILE : WAVES * MAXRB * OB;
 };
 
+// Normalises row block r of a wave (lane (g, n) holds O rows 4g + i, columns
+// 16j + n, and l of row n) and stages it at `ob` for the output stores (see
+// the end of the run kernel).
 template <int D, int MAXRB>
-__global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_eu(D <= 128 ? PREFILL_WAVES : 1))) void prefill_run_kernel(RunParams p) {
+__device__ __forceinline__ void stage_rows(lds_t* ob, int r, int lane, const mi::f32x4_t (&o)[D / 16], float lt) {
   using T = PrefillTraits<D, MAXRB>;
-  __shared__ __attribute__((aligned(16))) char smem[T::SMEM];  // [buffer][K, V], then the output rows
-  lds_t* lds = (lds_t*)smem;
+  const int g = lane >> 4, n = lane & 15;
+  const int wcol = n * 32 + (n >> 3) * kOutPad + 8 * g;
+  float inv[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float li = mi::lane_shuffle(lt, 4 * g + i);
+    inv[i] = li > 0.f ? mi::fast_rcp(li) : 0.f;
+  }
+#pragma unroll
+  for (int j = 0; j < T::NT; ++j)  // column 16j + n: 8-column block 2j + n / 8
+    lds_store8(ob + r * T::OB + j * 2 * T::OUT_BLK + wcol,
+               u32x2_t{mi::cvt_pk_bf16(o[j][0] * inv[0], o[j][1] * inv[1]),
+                       mi::cvt_pk_bf16(o[j][2] * inv[2], o[j][3] * inv[3])});
+}
 
-  const int tile_idx = int(blockIdx.x) / p.hkv;
-  const int hkv = int(blockIdx.x) - tile_idx * p.hkv;
-  if (tile_idx >= p.header->num_tiles) return;  // whole workgroup
-  const PrefillTile t = p.tiles[tile_idx];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// Where the plan keeps the partials (PrefillHeader).
+struct PartialArea {
+  int64_t off;
+  int slots;
+};
+
+// Publishes a split unit's partial (O, m, l in fp32) and counts it; the last
+// of the tile's units reads all of them back in split order (so the result
+// does not depend on which came last), stages the merged rows for the output
+// stores and returns true.  The others return false.  Partials go through
+// device-coherent (sc1) stores and loads, as the units of a tile may run on
+// different XCDs; the counter is back at zero for the next run of the plan.
+// What bounds a merge is the round trip of its reads (104 KB per split at
+// head_dim 128): the wave walks (row block, split) as one sequence with DP
+// row blocks on their way.
+template <int D, int MAXRB>
+__device__ __forceinline__ bool merge_splits(const RunParams& p, int part, const PartialArea& pa, int hkv, int w, int lane, int nblk,
+                                             lds_t* lds, lds_t* ob, const mi::f32x4_t (&o)[MAXRB][D / 16],
+                                             const float (&m_run)[MAXRB], const float (&lt)[MAXRB]) {
+  using T = PrefillTraits<D, MAXRB>;
+  constexpr int NT = T::NT;
+  constexpr int CP = 16;  // cache policy: sc1 (device scope)
+  constexpr int DP = D == 256 ? 1 : MAXRB == 3 ? 3 : 4;
+  constexpr int WB = MAXRB * (NT * 1024 + 512);  // bytes of one wave's partial
+  static_assert(WB * T::WAVES == int(partial_bytes(D, MAXRB)), "partial layout");
+  const int g = lane >> 4;
+  const int nsplit = part & 0xff, split = (part >> 8) & 0xff, slot0 = int(unsigned(part) >> 16) - split;
+  char* base = p.ws + pa.off;
+  const int nslots = pa.slots;
+  // the wave's partial of split s, one descriptor each: the slots of one tile
+  // and KV head lie hkv slots apart
+  auto rsrc = [&](int s) {
+    char* a = base + (int64_t(slot0 + s) * p.hkv + hkv) * int64_t(WB * T::WAVES) + w * WB;
+    return __builtin_amdgcn_make_buffer_rsrc(a, (short)0, WB, kBufferWord3);
+  };
+  {
+    const __amdgpu_buffer_rsrc_t rs = rsrc(split);
+#pragma unroll
+    for (int r = 0; r < MAXRB; ++r) {
+      if (r >= nblk) continue;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, o[r][j]), rs, lane * 16, (r * NT + j) * 1024, CP);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{__float_as_uint(m_run[r]), __float_as_uint(lt[r])}, rs, lane * 8,
+                                            MAXRB * NT * 1024 + r * 512, CP);
+    }
+  }
+  // every wave's stores are acknowledged before one lane counts the unit
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+  __syncthreads();
+  int* counter = reinterpret_cast<int*>(base + int64_t(nslots) * p.hkv * int64_t(WB * T::WAVES)) +
+                 (int64_t(slot0) * p.hkv + hkv) * kCounterStride;
+  __attribute__((address_space(3))) int* flag = (__attribute__((address_space(3))) int*)lds;
+  if (threadIdx.x == 0) *flag = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int prev = __builtin_amdgcn_readfirstlane(*flag);
+  __syncthreads();  // the flag's bytes are staged over below
+  if (prev != nsplit - 1) return false;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  if (threadIdx.x == 0) __hip_atomic_store(counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+  u32x4_t v[DP][NT];
+  u32x2_t ml[DP];
+  const int steps = nblk * nsplit;
+  int rl = 0, sl = 0;  // the next step to load
+  auto load = [&](int q) {
+    const __amdgpu_buffer_rsrc_t rs = rsrc(sl);
+    ml[q] = __builtin_amdgcn_raw_buffer_load_b64(rs, lane * 8, MAXRB * NT * 1024 + rl * 512, CP);
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      v[q][j] = __builtin_amdgcn_raw_buffer_load_b128(rs, lane * 16, (rl * NT + j) * 1024, CP);
+    if (++sl == nsplit) {
+      sl = 0;
+      ++rl;
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < DP; ++q)
+    if (q < steps) load(q);
+  mi::f32x4_t acc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) acc[j] = mi::f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  int r = 0, s = 0;
+  for (int k = 0; k < steps; k += DP) {
+#pragma unroll
+    for (int q = 0; q < DP; ++q) {
+      if (k + q >= steps) break;
+      // row n of the block: the weights of what is merged so far and of this
+      // split (0 for a split that saw no key of the row: its m is -inf)
+      const float ms = __uint_as_float(ml[q].x), ls = __uint_as_float(ml[q].y);
+      const float mn = fmaxf(m, ms);
+      const float f0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+      const float f1 = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mn);
+      m = mn;
+      l = l * f0 + ls * f1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a0 = mi::lane_shuffle(f0, 4 * g + i), a1 = mi::lane_shuffle(f1, 4 * g + i);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[j][i] = acc[j][i] * a0 + __uint_as_float(v[q][j][i]) * a1;
+      }
+      if (k + q + DP < steps) load(q);
+      if (++s == nsplit) {
+        stage_rows<D, MAXRB>(ob, r, lane, acc, l);
+        m = -INFINITY;
+        l = 0.f;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[j] = mi::f32x4_t{0.f, 0.f, 0.f, 0.f};
+        s = 0;
+        ++r;
+      }
+    }
+  }
+  return true;
+}
+
+// One unit of the run (a workgroup), MAXRB row blocks per wave.
+template <int D, int MAXRB>
+__device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& t, const PartialArea& pa, int hkv, int bm,
+                                         lds_t* lds) {
+  using T = PrefillTraits<D, MAXRB>;
+  const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, n = lane & 15;
   const int off = t.kv_len - t.qo_len;
   // the workgroup's rows in position-major order: row R is position R / group
   // of the tile, head R % group of this KV head's group; row block rb holds
   // rows 16 rb .. 16 rb + 15
-  const int nrows = p.bm * p.group;
+  const int nrows = bm * p.group;
   const int nrb = (nrows + 15) / 16;
-
 
   // ---- this wave's row blocks: rb = w, w + 4
   mi::bf16x8_t qb[T::MAXRB][T::KSTEPS];
@@ -349,10 +764,14 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
 #pragma unroll
   for (int r = 0; r < T::MAXRB; ++r)
     if (qpos[r] >= 0) qmin = min(qmin, qpos[r]);
-  qmin = -wave_max_i(-qmin);
+  qmin = __builtin_amdgcn_readfirstlane(-wave_max_i(-qmin));
   int block_hi = p.causal ? min(t.kv_len, t.row0 + t.q_rows + off) : t.kv_len;
   block_hi = max(block_hi, 0);
-  const int ntile = (block_hi + kKvTile - 1) / kKvTile;
+  // this unit's KV tiles (a split tile's last unit takes all that remain)
+  const int nsplit = t.part & 0xff;
+  const int ntile = __builtin_amdgcn_readfirstlane(min((block_hi + kKvTile - 1) / kKvTile,
+      unsigned(t.kt) >> 16 == kToEnd ? 0x7fffffff : int(unsigned(t.kt) >> 16)));
+  const int kt0 = t.kt & 0xffff;
 
   // ---- staging.  Load i of a thread covers token ltok + TPL i of the tile
   // and 16-byte chunk ldc of that token's row: a wave's 64 lanes cover whole
@@ -374,10 +793,9 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
   // chunk_slot(row, slot) (the permutation is its own inverse); a block lies
   // inside one page, so the page index is wave-uniform.
   constexpr int RPB = 1024 / (D * 2);
-  const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
 #pragma unroll
   for (int i = 0; i < T::LOADS; ++i) {
-    const int bk = T::WAVES * i + wv;
+    const int bk = T::WAVES * i + w;
     const int tr = bk * RPB + lane / T::CPR;
     pit[i] = __builtin_amdgcn_readfirstlane(bk * RPB / kPageSize);
     voff[i] = (tr % kPageSize) * tok_bytes + hkv * D * 2 + chunk_slot<D>(tr, lane % T::CPR) * 16;
@@ -402,23 +820,24 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
 #pragma unroll
     for (int i = 0; i < T::LOADS; ++i) {
       const int pg_idx = kt * (kKvTile / kPageSize) + pit[i];
-      // the index is clamped into the request's pages (it has >= 1 page
-      // whenever there is a tile), then the id is dropped past the end
-      const int v = kv_ids[t.kv_page_begin + min(pg_idx, npages_req - 1)];
-      pid[i] = (kt < ntile && pg_idx < npages_req) ? v : -1;
+      // clamped into the request's pages (it has >= 1 page whenever there is
+      // a tile); an id past the end is dropped when it is used, so that
+      // nothing here waits for these loads (with the test beside them each of
+      // the loads was waited for in turn)
+      pid[i] = kv_ids[t.kv_page_begin + min(pg_idx, npages_req - 1)];
     }
   };
   auto load_tile = [&](int kt, int buf) {
 #pragma unroll
     for (int i = 0; i < T::LOADS; ++i) {
-      const int pg = pid[i];
-      const bool ok = pg >= 0 && pg < p.num_pages;
+      const int pg = __builtin_amdgcn_readfirstlane(pid[i]);
       const int pg_idx = kt * (kKvTile / kPageSize) + pit[i];
+      const bool ok = unsigned(pg) < p.num_pages && pg_idx < npages_req;
       const int size = !ok ? 0 : (pg_idx == npages_req - 1 ? kv_bytes + last_rows * tok_bytes : page_bytes);
       const char* base = reinterpret_cast<const char*>(p.pool) + (ok ? int64_t(pg) * page_bytes : 0);
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, size, kBufferWord3);
 #if PREFILL_DMA
-      lds_t* kdst = lds + buf * 2 * T::TILE + 1024 * (T::WAVES * i + wv);
+      lds_t* kdst = lds + buf * 2 * T::TILE + 1024 * (T::WAVES * i + w);
       lds_dma16(rs, kdst, voff[i], 0);
       lds_dma16(rs, kdst + T::TILE, voff[i], kv_bytes);
 #else
@@ -442,10 +861,10 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
 #endif
   };
 
-  if (ntile > 0) {
-    fetch_ids(0);
-    load_tile(0, 0);
-    fetch_ids(1);
+  if (kt0 < ntile) {
+    fetch_ids(kt0);
+    load_tile(kt0, 0);
+    fetch_ids(kt0 + 1);
     store_tile(0);
   }
   // Everything loaded so far (Q, tile 0, the next page ids) is waited for
@@ -470,8 +889,8 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
                               : vr * T::RS + (n & 3) * 8 + 32 * j;
   }
 
-  for (int kt = 0; kt < ntile; ++kt) {
-    const int buf = kt & 1;
+  for (int kt = kt0; kt < ntile; ++kt) {
+    const int buf = (kt - kt0) & 1;
     if (kt + 1 < ntile) {
       load_tile(kt + 1, buf ^ 1);
       fetch_ids(kt + 2);
@@ -496,10 +915,10 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
       // so full tiles carry no mask code), the row maxima, one lazy-rescale
       // branch for the wave, then exp / pack / P V half by half, so the P V
       // MFMAs of keys 0-31 can overlap the exponentials of keys 32-63.
-      float sv[T::MAXRB][4][4];
+      float sv[T::MAXRB][kKvTile / 16][4];
       auto scores = [&](auto masked) {
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
+        for (int kb = 0; kb < kKvTile / 16; ++kb) {
           mi::bf16x8_t ka[T::KSTEPS];
 #pragma unroll
           for (int s = 0; s < T::KSTEPS; ++s)
@@ -540,7 +959,7 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
         for (int r = 0; r < T::MAXRB; ++r) {
           float m = sv[r][0][0];
 #pragma unroll
-          for (int kb = 0; kb < 4; ++kb)
+          for (int kb = 0; kb < kKvTile / 16; ++kb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) m = fmaxf(m, sv[r][kb][i]);
           mloc[r] = max_xor32(max_xor16(m)) * p.scale_log2;  // scale > 0 keeps the arg max
@@ -568,7 +987,7 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
           }
         }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < kKvTile / 32; ++h) {
           // exp2(-inf - m) = 0 for masked keys; m is taken as 0 while the row
           // has seen no key (m_run still -inf), avoiding -inf - -inf
           mi::bf16x8_t pa[T::MAXRB];
@@ -661,23 +1080,17 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
   constexpr int kOutBlk = T::OUT_BLK;
   constexpr int OB = T::OB;
   lds_t* const ob = lds + w * T::MAXRB * OB;
-  const int wcol = n * 32 + (n >> 3) * kOutPad + 8 * g;
+  float lt[T::MAXRB];
 #pragma unroll
-  for (int r = 0; r < T::MAXRB; ++r) {
-    if (r >= nblk) continue;
-    const float lt = sum_xor32(sum_xor16(l_run[r]));
-    float inv[4];
+  for (int r = 0; r < T::MAXRB; ++r) lt[r] = sum_xor32(sum_xor16(l_run[r]));
+  // Every unit stages its own rows first, a split one for nothing: `o` is then
+  // dead once a partial is published, whichever way the unit goes on, and the
+  // merge has its registers for reads in flight.
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float li = mi::lane_shuffle(lt, 4 * g + i);
-      inv[i] = li > 0.f ? mi::fast_rcp(li) : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < T::NT; ++j)  // column 16j + n: 8-column block 2j + n / 8
-      lds_store8(ob + r * OB + j * 2 * kOutBlk + wcol,
-                 u32x2_t{mi::cvt_pk_bf16(o[r][j][0] * inv[0], o[r][j][1] * inv[1]),
-                         mi::cvt_pk_bf16(o[r][j][2] * inv[2], o[r][j][3] * inv[3])});
-  }
+  for (int r = 0; r < T::MAXRB; ++r)
+    if (r < nblk) stage_rows<D, MAXRB>(ob, r, lane, o[r], lt[r]);
+  if (nsplit > 1 && !merge_splits<D, MAXRB>(p, t.part, pa, hkv, w, lane, nblk, lds, ob, o, m_run, lt))
+    return;
   __syncthreads();
   const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
       (void*)(p.out + int64_t(t.q_begin) * p.o_st), (short)0,
@@ -698,6 +1111,32 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
           __builtin_bit_cast(u32x4_t, (s16x8_t){a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]}), ro, off, 64 * q, 0);
     }
   }
+}
+
+// The plan says which form its tiles have: coarse, RB row blocks per wave, or
+// fine, one.
+template <int D, int RB>
+__global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void prefill_run_kernel(RunParams p) {
+  __shared__ __attribute__((aligned(16))) char smem[PrefillTraits<D, RB>::SMEM];  // [buffer][K, V], then the output rows
+  static_assert(PrefillTraits<D, 1>::SMEM <= PrefillTraits<D, RB>::SMEM, "LDS of the fine form");
+  lds_t* lds = (lds_t*)smem;
+  const int tile_idx = int(blockIdx.x) / p.hkv;
+  const int hkv = int(blockIdx.x) - tile_idx * p.hkv;
+  // The header and the record (not written during the launch) are read through
+  // the constant address space, so they arrive in scalar registers: as vector
+  // loads, which the stores of partials otherwise make of them, the compiler
+  // put a per-lane loop around every page load of head_dim 256 (2.9 -> 3.3 us
+  // per KV tile).
+  typedef __attribute__((address_space(4))) const PrefillHeader const_header;
+  typedef __attribute__((address_space(4))) const int const_int;
+  const const_header* h = (const const_header*)(p.header);
+  if (tile_idx >= h->num_tiles) return;  // whole workgroup
+  const const_int* f = (const const_int*)(p.tiles + tile_idx);
+  const PrefillTile t{f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
+  const PartialArea pa{h->split_off, h->slots};
+  const int bm = h->bm;
+  if (RB > 1 && h->row_blocks == 1) run_unit<D, 1>(p, t, pa, hkv, bm, lds);
+  else run_unit<D, RB>(p, t, pa, hkv, bm, lds);
 }
 
 }  // namespace
@@ -731,10 +1170,22 @@ extern "C" int mi_prefill_plan(void* workspace, size_t workspace_bytes, const in
   pp.last_page_len = kv_last_page_len;
   pp.batch = batch_size;
   pp.capacity = int(tile_capacity(batch_size, total_q));
-  pp.bm = rows_per_tile(num_qo_heads / num_kv_heads, head_dim);
+  pp.group = num_qo_heads / num_kv_heads;
+  pp.hkv = num_kv_heads;
+  pp.resident = resident_groups(head_dim);
+  const PartialLayout L = partial_layout(workspace_bytes, num_kv_heads, head_dim);
+  pp.split_off = int64_t(L.off);
+  pp.split_capacity = L.coarse ? int(std::min<size_t>((L.off - 256) / sizeof(PrefillTile), 1 << 30)) : 0;
+  for (int form = 0; form < 2; ++form) {
+    pp.blocks[form] = form ? row_blocks(head_dim) : 1;
+    pp.bm[form] = rows_per_tile(pp.group, head_dim, pp.blocks[form]);
+    pp.slots[form] = form ? L.coarse : L.fine;
+    pp.counters_off[form] = L.off + size_t(pp.slots[form]) * num_kv_heads * partial_bytes(head_dim, pp.blocks[form]);
+  }
+  pp.ws = ws;
   pp.header = reinterpret_cast<PrefillHeader*>(ws);
   pp.tiles = reinterpret_cast<PrefillTile*>(ws + 256);
-  hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(1024), 0, static_cast<hipStream_t>(stream), pp);
+  hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(kPlanThreads), 0, static_cast<hipStream_t>(stream), pp);
   return mi::check_launch("prefill_plan_kernel");
 }
 
@@ -764,17 +1215,18 @@ extern "C" int mi_prefill_run(void* workspace, size_t workspace_bytes, const voi
     return mi::fail(MI_ERR_INVALID, "prefill run: q rows, out rows and pool must be 16-byte aligned");
   if (q_stride_token < 0 || q_stride_head < 0 || out_stride_token < 0 || out_stride_head < 0)
     return mi::fail(MI_ERR_INVALID, "prefill run: negative stride");
-  const int64_t grid = int64_t(tile_capacity(batch_size, total_q)) * num_kv_heads;
+  const int64_t grid = run_groups(batch_size, total_q, num_qo_heads / num_kv_heads, num_kv_heads, head_dim);
   if (grid > 0x7fffffff) return mi::fail(MI_ERR_INVALID, "prefill run: too many tiles");
   char* ws = static_cast<char*>(workspace);
   RunParams rp;
+  rp.ws = ws;
   rp.header = reinterpret_cast<const PrefillHeader*>(ws);
   rp.tiles = reinterpret_cast<const PrefillTile*>(ws + 256);
   rp.q = static_cast<const uint16_t*>(q);
   rp.q_st = q_stride_token;
   rp.q_sh = q_stride_head;
   rp.pool = static_cast<const uint16_t*>(paged_kv_cache);
-  rp.num_pages = num_pages;
+  rp.num_pages = unsigned(std::min<int64_t>(std::max<int64_t>(num_pages, 0), 0x7fffffff));
   rp.indices = kv_indices;
   rp.out = static_cast<uint16_t*>(out);
   rp.o_st = out_stride_token;
@@ -783,14 +1235,14 @@ extern "C" int mi_prefill_run(void* workspace, size_t workspace_bytes, const voi
   rp.hkv = num_kv_heads;
   rp.group = num_qo_heads / num_kv_heads;
   rp.causal = causal ? 1 : 0;
-  rp.bm = rows_per_tile(rp.group, head_dim);
+  const int bm = rows_per_tile(rp.group, head_dim, row_blocks(head_dim));
   // a tile addresses its q / out rows through one buffer descriptor each, by
   // 32-bit byte offsets from its first position: any strides (heads inside a
   // position's row, or head-major) whose tile extent fits
   rp.q_ext = int64_t(num_qo_heads - 1) * q_stride_head + head_dim;
   rp.o_ext = int64_t(num_qo_heads - 1) * out_stride_head + head_dim;
-  const int64_t q_span = (int64_t(rp.bm) - 1) * q_stride_token + rp.q_ext;
-  const int64_t o_span = (int64_t(rp.bm) - 1) * out_stride_token + rp.o_ext;
+  const int64_t q_span = (int64_t(bm) - 1) * q_stride_token + rp.q_ext;
+  const int64_t o_span = (int64_t(bm) - 1) * out_stride_token + rp.o_ext;
   if (q_span > 0x3fffffff || o_span > 0x3fffffff)
     return mi::fail(MI_ERR_INVALID, "prefill run: q / out strides span %lld / %lld elements per tile (at most 2^30)",
                     (long long)q_span, (long long)o_span);

@@ -232,3 +232,51 @@ def test_long_prompt_4096(dev, parity):
     b = make_paged_batch([4096], 8, 2, 128, seed=41)
     out, ref = _run(dev, b, [4096], 8, 2, 128, seed=41)
     parity(out, ref)
+
+
+# (heads, new rows per request, cached tokens per request, row blocks per wave the plan picks)
+SPLIT_CASES = [
+    ((32, 8, 128), [3], [1000], 1),             # one short tile per KV head, cut at kMinChunk
+    ((28, 4, 128), [193, 1, 64], [900, 65, 0], 1),  # fine tiles, ragged, one that is not split
+    ((8, 1, 64), [2], [9000], 1),               # a single tile: the most units one merge takes
+    ((64, 8, 128), [200, 37], [5001, 3000], 3),  # coarse tiles of three row blocks
+    ((14, 2, 64), [700], [4010], 2),
+    ((16, 4, 256), [70], [2500], 1),
+]
+
+
+@pytest.mark.parametrize("heads,qo_lens,cached,blocks", SPLIT_CASES)
+@pytest.mark.parametrize("causal", [True, False])
+def test_tiles_split_over_the_keys(dev, parity, heads, qo_lens, cached, blocks, causal):
+    """Tiles cut into units along the keys: against the oracle, the same bits
+    on every run of a plan (the merge counters are back at zero), and with a
+    workspace that has no room for partials (nothing is split)."""
+    from minimal_inference_amd import _lib
+    from minimal_inference_amd.prefill import BatchPrefillWithPagedKVCacheWrapper
+
+    hq, hkv, d = heads
+    b = make_paged_batch([q + c for q, c in zip(qo_lens, cached)], hq, hkv, d, seed=17)
+    total = sum(qo_lens)
+    q = torch.randn(total, hq, d, generator=torch.Generator().manual_seed(17)).to(torch.bfloat16)
+    qo = [0]
+    for n in qo_lens:
+        qo.append(qo[-1] + n)
+    args = [torch.tensor(qo, dtype=torch.int32, device=dev), torch.tensor(b["indptr"], dtype=torch.int32, device=dev),
+            b["indices"].to(dev), torch.tensor(b["last"], dtype=torch.int32, device=dev)]
+    qd, pool = q.to(dev), b["pool"].to(dev)
+    ref = oatt.prefill(q, b["pool"], qo, b["indptr"], b["indices"].tolist(), b["last"], causal=causal)
+
+    def run(nbytes):
+        ws = torch.full((nbytes,), 0x5a, dtype=torch.uint8, device=dev)
+        w = BatchPrefillWithPagedKVCacheWrapper(ws, "NHD")
+        w.plan(*args, hq, hkv, d, 16, causal=causal, max_total_q=total)
+        outs = [w.run(qd, pool).cpu() for _ in range(3)]
+        return ws[:32].view(torch.int32).tolist(), outs
+
+    header, outs = run(128 << 20)
+    assert header[1] == 0 and header[3] == blocks and header[4] > 0  # no error, the form, a split
+    parity(outs[0].float(), ref)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    header, whole = run(int(_lib.load().mi_prefill_workspace_size(len(qo_lens), total)))
+    assert header[1] == 0 and header[4] == 0
+    parity(whole[0].float(), ref)
