@@ -1,16 +1,18 @@
-"""Fused dense-layer helpers: residual add + RMSNorm, SiLU-gated product.
+"""Dense-layer helpers: residual add + RMSNorm, SiLU-gated product, few-row linear.
 
 ``add_rms_norm(x, delta, weight, eps)`` stands for ``x = x + delta`` followed
 by ``F.rms_norm(x, (H,), weight, eps)`` (DecoderLayer.forward,
 model.py:324-344; RMSNorm, model.py:115-122); ``silu_mul(gate_up)`` for
 ``F.silu(gate) * up`` over the fused gate/up projection (MLP,
 model.py:301-311).  Both run one HIP kernel (``mi_add_rms_norm`` /
-``mi_silu_mul``); there is no torch fallback.
+``mi_silu_mul``); there is no torch fallback.  ``linear(x, weight, bias)`` is
+``F.linear`` with a decode step's few rows on ``mi_linear``.
 """
 
 from __future__ import annotations
 
 import torch
+import torch.nn.functional as F
 
 from . import _lib
 from ._util import require_dtype, require_gpu, stream_of
@@ -67,4 +69,39 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Te
     _rows("out", out, inter)
     _lib.call("mi_silu_mul", gate_up.data_ptr(), gate_up.stride(0), out.data_ptr(), out.stride(0), rows, inter,
               stream_of(gate_up))
+    return out
+
+
+# Most rows the few-row kernel takes.
+LINEAR_MAX_ROWS = 32
+
+
+def _few_rows(rows: int, n: int, k: int) -> bool:
+    """Whether the few-row kernel is the faster one: up to 16 rows everywhere but on
+    the largest weights of long rows (59,136 x 8,192, 16 rows: 181 us, library 170),
+    up to 32 while k is short (4,096 x 14,336: 34 us, library 31; 28,672 x 4,096:
+    46 us, library 55)."""
+    if rows <= 16:
+        return k < 8192 or n <= 32768
+    return rows <= LINEAR_MAX_ROWS and k < 8192
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """``F.linear`` of [rows, k]; a decode step's few rows of bf16 go to the kernel
+    that streams the weight once (fp32 accumulation, one rounding), everything else
+    to torch."""
+    rows, k = x.shape
+    n = weight.shape[0]
+    if (rows == 0 or not _few_rows(rows, n, k) or n % 16 or k % 64 or not x.is_cuda
+            or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device
+            or weight.shape[1] != k or not weight.is_contiguous() or x.stride(1) != 1 or x.stride(0) % 8
+            or x.stride(0) < k or x.data_ptr() % 16 or weight.data_ptr() % 16
+            or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+            or (bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (n,) or not bias.is_contiguous()
+                                      or bias.device != x.device or bias.data_ptr() % 8
+                                      or (torch.is_grad_enabled() and bias.requires_grad)))):
+        return F.linear(x, weight, bias)
+    out = torch.empty(rows, n, dtype=x.dtype, device=x.device)
+    _lib.call("mi_linear", x.data_ptr(), x.stride(0), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
+              out.data_ptr(), n, rows, n, k, stream_of(x))
     return out

@@ -2,8 +2,8 @@
 
 Restates model.py of the reference (ModelConfig 37-71, RoPE 79-107, RMSNorm
 115-122, Attention 126-252, MLP 301-311, DecoderLayer 314-344, Model
-352-435).  Dense GEMMs, RMSNorm and RoPE stay on PyTorch-ROCm (hipBLASLt);
-the attention layer calls the HIP library through the reference's drop-in
+352-435).  The GEMMs of many rows stay on PyTorch-ROCm (hipBLASLt); the
+attention layer calls the HIP library through the reference's drop-in
 surface: ``append_paged_kv_cache`` then ``wrapper.run`` (model.py:207-235),
 without the reference's Q-head padding (model.py:134-137, 226-243): any
 integer GQA group runs natively.
@@ -19,9 +19,10 @@ separate launch), bit-identical again; ``fused_rope=False`` keeps the
 separate ops.
 By default the residual adds and the RMSNorms that follow them run as one
 HIP kernel each, and SiLU(gate) * up as one (``dense.add_rms_norm`` /
-``dense.silu_mul``, fp32 math, one bf16 rounding per output);
-``fused_dense=False`` keeps torch's ``F.rms_norm``, adds and
-``F.silu(g) * u``.  RoPE tables are held in the model dtype, as the reference's are after ``.to(dtype)``
+``dense.silu_mul``, fp32 math, one bf16 rounding per output), and the
+projections of a decode step's few rows on the kernel that streams each weight
+once (``dense.linear``); ``fused_dense=False`` keeps torch's ``F.linear``,
+``F.rms_norm``, adds and ``F.silu(g) * u``.  RoPE tables are held in the model dtype, as the reference's are after ``.to(dtype)``
 (server.py:251).  Weights are random-initialised on the device (N(0, 0.02),
 norms 1) -- the benchmark configurations use random weights.
 """
@@ -36,7 +37,7 @@ import os
 import torch
 import torch.nn.functional as F
 
-from .dense import add_rms_norm, silu_mul
+from .dense import add_rms_norm, linear, silu_mul
 from .page import append_paged_kv_cache, rope_append_paged_kv_cache
 
 
@@ -207,13 +208,14 @@ class Model:
         backend._layer_idx = 0
         eps = cfg.rms_norm_eps
         dense = self.fused_dense
+        project = linear if dense else F.linear
         if dense:
             h = add_rms_norm(x, None, self.layers[0].in_norm, eps, write_x=False)
         for li, L in enumerate(self.layers):
             layer_idx = backend.next_layer()
             if not dense:
                 h = F.rms_norm(x, (cfg.hidden_size,), L.in_norm, eps)
-            qkv = F.linear(h, L.w_qkv, L.b_qkv)
+            qkv = project(h, L.w_qkv, L.b_qkv)
             kv_data = backend.paged_kv_cache.kv_data[layer_idx]
             if fused and backend.mode == "decode" and self.fused_decode:
                 # RoPE, append and attention in one launch (one new token per
@@ -240,8 +242,8 @@ class Model:
                 x = x + F.linear(F.silu(g) * u, L.w_down)
                 continue
             # x += o W_o; h = rms(x); x += down(silu(g) * u); h = next layer's rms(x)
-            h = add_rms_norm(x, F.linear(o.view(t, nq * d), L.w_o), L.post_norm, eps)
-            down = F.linear(silu_mul(F.linear(h, L.w_gate_up)), L.w_down)
+            h = add_rms_norm(x, project(o.view(t, nq * d), L.w_o), L.post_norm, eps)
+            down = project(silu_mul(project(h, L.w_gate_up)), L.w_down)
             if li + 1 < len(self.layers):
                 h = add_rms_norm(x, down, self.layers[li + 1].in_norm, eps)
             elif last_rows is None:
@@ -253,7 +255,7 @@ class Model:
             if last_rows is not None:
                 x = x.index_select(0, last_rows)
             h = F.rms_norm(x, (cfg.hidden_size,), self.norm, eps)
-        return F.linear(h, self.lm_head)
+        return project(h, self.lm_head)
 
 
 def kv_pool_bytes_per_page(cfg: ModelConfig, page_size: int = 16) -> int:

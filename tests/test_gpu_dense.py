@@ -122,3 +122,62 @@ def test_model_prefill_logits_fused_vs_unfused(dev):
         logits.append(captured["l"].float())
     rel = (logits[0] - logits[1]).abs().max().item() / logits[1].abs().max().item()
     assert rel < 2e-2, rel
+
+
+@pytest.mark.parametrize("rows", [1, 8, 15, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [
+    (16, 64), (48, 192), (1152, 896), (896, 4864), (4096, 320),   # one tile per workgroup, few slabs, odd slab counts
+    (4112, 4096), (8176, 128), (8208, 576),                       # either side of 256 and 512 tiles of 16 columns
+    (32768, 256), (32800, 256), (151936, 896),                    # 2,048 tiles, past them with a partial last workgroup
+    (512, 8192), (16, 18944),                                     # long rows
+])
+def test_few_row_linear(dev, rows, n, k):
+    """mi_linear at the edges of its forms against an fp32 product of the same
+    bf16 values; x rows and out rows strided, and the columns and rows around
+    them untouched.
+
+    Bound: the sum of k products in fp32, in any order, is within
+    k * 2^-24 * sum |x w| of the exact one, and the result is rounded once to
+    bf16 (2^-8 relative); the reference's own fp32 error is of the first kind."""
+    from minimal_inference_amd import _lib
+
+    g = torch.Generator(device=dev).manual_seed(rows * 131 + n + k)
+    big = torch.randn(rows, k + 64, device=dev, generator=g).to(torch.bfloat16)
+    x = big[:, 32:32 + k]
+    w = torch.randn(n, k, device=dev, generator=g).to(torch.bfloat16)
+    for bias in (None, torch.randn(n, device=dev, generator=g).to(torch.bfloat16)):
+        out = torch.full((rows + 1, n + 8), 7.0, device=dev, dtype=torch.bfloat16)
+        _lib.call("mi_linear", x.data_ptr(), x.stride(0), w.data_ptr(), bias.data_ptr() if bias is not None else None,
+                  out.data_ptr(), out.stride(0), rows, n, k, torch.cuda.current_stream().cuda_stream)
+        b = 0.0 if bias is None else bias.float()
+        ref = x.float() @ w.float().t() + b
+        mag = x.float().abs() @ w.float().abs().t() + (0.0 if bias is None else bias.float().abs())
+        err = (out[:rows, :n].float() - ref).abs()
+        assert bool((err <= 2 ** -8 * ref.abs() + 2 * k * 2 ** -24 * mag).all())
+        assert bool((out[rows] == 7.0).all()) and bool((out[:, n:] == 7.0).all())
+        again = torch.empty_like(out)
+        _lib.call("mi_linear", x.data_ptr(), x.stride(0), w.data_ptr(), bias.data_ptr() if bias is not None else None,
+                  again.data_ptr(), again.stride(0), rows, n, k, torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(again[:rows, :n], out[:rows, :n])
+
+
+def test_few_row_linear_routes(dev):
+    """dense.linear: the kernel and torch's F.linear agree to bf16 rounding where
+    the kernel takes the call, and the calls it does not take (more rows, odd
+    widths, other types and layouts, gradients) are F.linear's, bit for bit."""
+    from minimal_inference_amd.dense import linear
+
+    x = torch.randn(8, 512, device=dev).to(torch.bfloat16)
+    w = torch.randn(256, 512, device=dev).to(torch.bfloat16)
+    b = torch.randn(256, device=dev).to(torch.bfloat16)
+    assert _ulp_close(linear(x, w, b), F.linear(x.float(), w.float(), b.float()).to(torch.bfloat16), 1)
+    assert linear(x[:0], w).shape == (0, 256)
+    for xx, ww in [(x.repeat(5, 1), w), (x[:, :480], w[:, :480]), (x[:, :480], w[:, :480].contiguous()),
+                   (x, w[:250]), (x.float(), w.float()), (x.t().contiguous().t(), w)]:
+        assert torch.equal(linear(xx, ww), F.linear(xx, ww))
+    wg = w.clone().requires_grad_()
+    linear(x, wg).float().sum().backward()
+    assert wg.grad is not None
+    with pytest.raises(ValueError):
+        from minimal_inference_amd import _lib
+        _lib.call("mi_linear", x.data_ptr(), 512, w.data_ptr(), None, b.data_ptr(), 256, 33, 256, 512, 0)
