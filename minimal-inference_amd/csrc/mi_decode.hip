@@ -704,15 +704,29 @@ __device__ __forceinline__ void decode_unit(const RunParams& p, int u, int iv, l
   auto wg_sync = [&]() {
     if constexpr (W > 1) __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   };
-  auto scores = [&](int which, int valid, float (&sv)[4]) {
-    const lds_t* kl = k_slot(which);
-    mi::f32x4_t c = {0.f, 0.f, 0.f, 0.f};
+  // S^T of both pages.  All of the K operand reads go out before the first
+  // MFMA (and likewise the V reads below): left alone, the scheduler
+  // saved registers by waiting for the LDS read of each MFMA in turn, and a
+  // pair's chain of some 16 read latencies, ~1.7 us, set the pace wherever
+  // memory did not.
+  auto scores = [&](int va, int vb, float (&sa)[4], float (&sb)[4]) {
+    mi::bf16x8_t ka[2][T::KSTEPS];
 #pragma unroll
     for (int s = 0; s < T::KSTEPS; ++s)
-      c = mi::mfma_16x16x32_bf16(__builtin_bit_cast(mi::bf16x8_t, lds_load16(kl + j * T::RS + (g + 4 * s) * 16)),
-                                 qb[s], c);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sv[i] = (4 * g + i < valid) ? c[i] * p.scale_log2 : -INFINITY;
+      for (int h = 0; h < 2; ++h)
+        ka[h][s] = __builtin_bit_cast(mi::bf16x8_t, lds_load16(k_slot(h) + j * T::RS + (g + 4 * s) * 16));
+    __builtin_amdgcn_sched_barrier(0);
+    mi::f32x4_t c[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int s = 0; s < T::KSTEPS; ++s)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) c[h] = mi::mfma_16x16x32_bf16(ka[h][s], qb[s], c[h]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sa[i] = (4 * g + i < va) ? c[0][i] * p.scale_log2 : -INFINITY;
+      sb[i] = (4 * g + i < vb) ? c[1][i] * p.scale_log2 : -INFINITY;
+    }
   };
   // `next` reloads the two staging register sets with the next pages as
   // soon as their rows are in LDS, so the loads of the next pair are in
@@ -737,8 +751,7 @@ __device__ __forceinline__ void decode_unit(const RunParams& p, int u, int iv, l
     wg_sync();
     if (ROPE && inj >= 0) inject(inj, last_valid - 1);
     float sa[4], sb[4];
-    scores(0, va, sa);
-    scores(1, vb, sb);
+    scores(va, vb, sa, sb);
     // ---- online softmax for head j, lazy rescale
     float mloc = fmaxf(fmaxf(fmaxf(sa[0], sa[1]), fmaxf(sa[2], sa[3])), fmaxf(fmaxf(sb[0], sb[1]), fmaxf(sb[2], sb[3])));
     mloc = max_xor16(mloc);
@@ -773,12 +786,21 @@ __device__ __forceinline__ void decode_unit(const RunParams& p, int u, int iv, l
     const mi::bf16x8_t pa = __builtin_bit_cast(
         mi::bf16x8_t,
         __builtin_convertvector((f32x8_v){pv[0], pv[1], pv[2], pv[3], pv[4], pv[5], pv[6], pv[7]}, bf16x8_v));
+    s16x4_t vx[T::NT], vy[T::NT];
+    {
+      const lds_t* va_row = v_slot(0) + (4 * g + (j >> 2)) * T::RS + (j & 3) * 8;
+      const lds_t* vb_row = v_slot(1) + (4 * g + (j >> 2)) * T::RS + (j & 3) * 8;
+#pragma unroll
+      for (int t = 0; t < T::NT; ++t) {
+        vx[t] = lds_read_tr16(va_row + 32 * t);
+        vy[t] = lds_read_tr16(vb_row + 32 * t);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     // ---- O += P V
-    const lds_t* va_row = v_slot(0) + (4 * g + (j >> 2)) * T::RS + (j & 3) * 8;
-    const lds_t* vb_row = v_slot(1) + (4 * g + (j >> 2)) * T::RS + (j & 3) * 8;
 #pragma unroll
     for (int t = 0; t < T::NT; ++t) {
-      const s16x4_t x = lds_read_tr16(va_row + 32 * t), y = lds_read_tr16(vb_row + 32 * t);
+      const s16x4_t x = vx[t], y = vy[t];
       const mi::bf16x8_t vbop = __builtin_bit_cast(mi::bf16x8_t, (s16x8_t){x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]});
       acc[t] = mi::mfma_16x16x32_bf16(pa, vbop, acc[t]);
     }
