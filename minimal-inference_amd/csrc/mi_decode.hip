@@ -263,6 +263,12 @@ __device__ __forceinline__ float group_sum(float x) {
 // chunk l % LR; the splits' m and l are laid out the same way (lane l: head
 // l / LR of a row group, split l % LR of a split group), so the weight of
 // split s for a lane's head is a shuffle inside its LR-lane group.
+//
+// More than direct_splits() of them merge in two levels (split_groups): the last
+// unit of a group merges the group as above, but publishes the sum, its m and
+// its l -- all fp32, the row's halves in the place of the group's first two
+// bf16 rows, which nobody reads any more -- and counts for the group; the last
+// group merges the groups.
 template <int D, int G>
 __device__ __forceinline__ void publish_merge(const RunParams& p, int u, int b, int hkv, int nsplit, int item_base,
                                               const mi::f32x4_t (&acc)[DecodeTraits<D, G>::NT], float m_run,
@@ -301,14 +307,22 @@ __device__ __forceinline__ void publish_merge(const RunParams& p, int u, int b, 
   // Wait until this wave's stores are acknowledged (vmcnt 0; expcnt /
   // lgkmcnt left free), so they are visible before the counter moves.  The
   // fence keeps the compiler from reordering around it.
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-  int prev = 0;
   int* counter = p.counters + (b * p.hkv + hkv) * kCounterStride;
-  if (lane == 0) prev = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  prev = mi::read_lane_i(prev, 0);
-  if (prev != nsplit - 1) return;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  auto count = [&](int* c) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    int prev = 0;
+    if (lane == 0) prev = __hip_atomic_fetch_add(c, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    prev = mi::read_lane_i(prev, 0);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    return prev;
+  };
+  // this unit's group: splits first .. first + n1 - 1
+  const int groups = split_groups(nsplit, direct_splits(D, G));
+  const int grp = groups == 1 ? 0 : ((u / p.hkv - item_base + 1) * groups - 1) / nsplit;
+  const int first = grp * nsplit / groups, n1 = (grp + 1) * nsplit / groups - first;
+  int* const my_counter = counter + (groups == 1 ? 0 : 1 + grp);
+  if (count(my_counter) != n1 - 1) return;
 
   constexpr int R = 1024 / (2 * D);   // rows per 16-byte load: 4 (D 128), 8 (D 64), 2 (D 256)
   constexpr int LR = 64 / R;          // lanes per row
@@ -325,11 +339,11 @@ __device__ __forceinline__ void publish_merge(const RunParams& p, int u, int b, 
 #pragma unroll
     for (int k = 0; k < 8; ++k) sum[a][k] = 0.f;
   }
-  auto unit_of = [&](int s) { return (item_base + s) * p.hkv + hkv; };
+  auto unit_of = [&](int s) { return (item_base + s) * p.hkv + hkv; };  // of split s of the request
   auto load_batch = [&](u32x4_t (&v)[KB][A], int s0, int nr) {
 #pragma unroll
     for (int q = 0; q < KB; ++q) {
-      const int us = unit_of(min(s0 + q, nr - 1));
+      const int us = unit_of(first + min(s0 + q, nr - 1));
 #pragma unroll
       for (int a = 0; a < A; ++a) {
         const int h = min(a * R + hg, G - 1);
@@ -337,14 +351,14 @@ __device__ __forceinline__ void publish_merge(const RunParams& p, int u, int b, 
       }
     }
   };
-  for (int r0 = 0; r0 < nsplit; r0 += 64) {
-    const int nr = min(64, nsplit - r0);
+  for (int r0 = 0; r0 < n1; r0 += 64) {
+    const int nr = min(64, n1 - r0);
     // (m, l) of split c LR + sg, head a R + hg; the first rows load with them
     typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
     u32x2_t ml[A][C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const int us = unit_of(r0 + min(c * LR + sg, nr - 1));
+      const int us = unit_of(first + r0 + min(c * LR + sg, nr - 1));
 #pragma unroll
       for (int a = 0; a < A; ++a)
         ml[a][c] = __builtin_amdgcn_raw_buffer_load_b64(rml, (us * G + min(a * R + hg, G - 1)) * 8, 0, CP);
@@ -454,6 +468,92 @@ __device__ __forceinline__ void publish_merge(const RunParams& p, int u, int b, 
       }
     }
   }
+  if (lane == 0) coherent_store(my_counter, 0);
+  if (groups > 1) {
+    const int u0 = unit_of(first), u1 = unit_of(first + 1);
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+      const int h = a * R + hg;
+      const int row = h < G ? h * D * 2 + sg * 16 : 0x7ffffff0 - u1 * G * D * 2;  // (lanes without a head store nowhere)
+      __builtin_amdgcn_raw_buffer_store_b128(
+          __builtin_bit_cast(u32x4_t, f32x4_v{sum[a][0], sum[a][1], sum[a][2], sum[a][3]}), rpo, u0 * G * D * 2 + row, 0, CP);
+      __builtin_amdgcn_raw_buffer_store_b128(
+          __builtin_bit_cast(u32x4_t, f32x4_v{sum[a][4], sum[a][5], sum[a][6], sum[a][7]}), rpo, u1 * G * D * 2 + row, 0, CP);
+      __builtin_amdgcn_raw_buffer_store_b64(
+          (__attribute__((ext_vector_type(2))) unsigned int){__float_as_uint(M[a]), __float_as_uint(Lt[a])}, rml,
+          h < G && sg == 0 ? (u0 * G + h) * 8 : 0x7ffffff0, 0, CP);
+    }
+    if (count(counter) != groups - 1) return;
+    // the groups' (m, l), laid out as the splits' above (at most 31 groups),
+    // and their rows, KG of them per round trip
+    typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
+    constexpr int KG = A == 1 ? 8 : A == 2 ? 4 : 2, C2 = (32 + LR - 1) / LR;
+    auto group_unit = [&](int q, int half) { return unit_of(min(q, groups - 1) * nsplit / groups + half); };
+    u32x4_t lo[KG][A], hi[KG][A];
+    auto load_groups = [&](int q0) {
+#pragma unroll
+      for (int q = 0; q < KG; ++q)
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+          const int row = min(a * R + hg, G - 1) * D * 2 + sg * 16;
+          lo[q][a] = __builtin_amdgcn_raw_buffer_load_b128(rpo, group_unit(q0 + q, 0) * G * D * 2 + row, 0, CP);
+          hi[q][a] = __builtin_amdgcn_raw_buffer_load_b128(rpo, group_unit(q0 + q, 1) * G * D * 2 + row, 0, CP);
+        }
+    };
+    u32x2_t ml[A][C2];
+#pragma unroll
+    for (int c = 0; c < C2; ++c)
+#pragma unroll
+      for (int a = 0; a < A; ++a)
+        ml[a][c] = __builtin_amdgcn_raw_buffer_load_b64(
+            rml, (group_unit(c * LR + sg, 0) * G + min(a * R + hg, G - 1)) * 8, 0, CP);
+    load_groups(0);
+    float wgt[A][C2];
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+      float mx = -INFINITY, ls = 0.f;
+#pragma unroll
+      for (int c = 0; c < C2; ++c)
+        if (c * LR + sg < groups) mx = fmaxf(mx, __uint_as_float(ml[a][c].x));
+      M[a] = group_max<LR>(mx);
+#pragma unroll
+      for (int c = 0; c < C2; ++c) {
+        const float ms = __uint_as_float(ml[a][c].x);
+        wgt[a][c] = (c * LR + sg < groups && ms != -INFINITY) ? __builtin_amdgcn_exp2f(ms - M[a]) : 0.f;
+        ls += wgt[a][c] * __uint_as_float(ml[a][c].y);
+      }
+      Lt[a] = group_sum<LR>(ls);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) sum[a][k] = 0.f;
+    }
+    static_assert(LR % KG == 0, "a round trip's groups share a weight register");
+#pragma nounroll
+    for (int q0 = 0; q0 < groups; q0 += KG) {
+      if (q0 > 0) load_groups(q0);
+      const int c0 = q0 / LR;
+      float wc[A];
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        wc[a] = wgt[a][0];
+#pragma unroll
+        for (int c = 1; c < C2; ++c) wc[a] = c0 == c ? wgt[a][c] : wc[a];
+      }
+#pragma unroll
+      for (int q = 0; q < KG; ++q) {
+        if (q0 + q >= groups) break;
+#pragma unroll
+        for (int a = 0; a < A; ++a) {
+          const float w = mi::lane_shuffle(wc[a], hg * LR + (q0 - c0 * LR) + q);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            sum[a][k] += w * __uint_as_float(lo[q][a][k]);
+            sum[a][4 + k] += w * __uint_as_float(hi[q][a][k]);
+          }
+        }
+      }
+    }
+    if (lane == 0) coherent_store(counter, 0);
+  }
   // lane (hg, sg) holds row positions 8 sg .. 8 sg + 7 of head a R + hg
 #pragma unroll
   for (int a = 0; a < A; ++a) {
@@ -468,7 +568,6 @@ __device__ __forceinline__ void publish_merge(const RunParams& p, int u, int b, 
       }
     }
   }
-  if (lane == 0) coherent_store(counter, 0);
 }
 
 // One unit: (item, KV head).  Lane l of the wave is (g, j) = (l >> 4, l & 15).
@@ -1075,6 +1174,7 @@ int mi::dplan::plan_setup(const char* who, void* workspace, size_t workspace_byt
   pp->hkv = hkv;
   pp->target_units = plan_target_units(batch, hq, hkv);
   pp->max_items = L.max_items;
+  pp->direct = direct_splits(head_dim, hq / hkv);
   pp->header = reinterpret_cast<DecodeHeader*>(ws);
   pp->items = reinterpret_cast<DecodeItem*>(ws + L.items);
   pp->counters = reinterpret_cast<int*>(ws + L.counters);

@@ -35,6 +35,24 @@ constexpr int kInlinePages = 24;
 // each, so the units' counting atomics on different counters do not queue on
 // one line.
 constexpr int kCounterStride = 32;
+// Groups that the splits of a (request, KV head) are merged in: more than
+// `direct` splits merge in two levels, near-equal groups first and then the
+// groups' results, since one wave reads 8 splits per round trip (a merge took
+// ~1.5 us + 0.14 us per split: 12.8 us of the 34 us that two requests of 16,001
+// and 32,001 tokens took on Qwen2.5-7B heads, 64 splits each).  A group counts
+// in the words behind the merge counter, in the same line.
+constexpr int kMaxGroups = kCounterStride - 1;
+__host__ __device__ constexpr int split_groups(int nsplit, int direct) {
+  if (nsplit <= direct) return 1;
+  const int per = nsplit <= 64 ? 8 : nsplit <= 256 ? 16 : 24;
+  const int n = (nsplit + per - 1) / per;
+  return n < kMaxGroups ? n : kMaxGroups;
+}
+// Three round trips while a 16-byte load per lane covers the rows of all of a
+// KV head's Q heads (19 splits, Mistral-7B heads B=4: direct 10.7 us, two
+// levels 11.0), two when it takes more loads (Qwen2.5-7B heads B=8, up to 24
+// splits: 13.8 and 13.1).
+__host__ __device__ constexpr int direct_splits(int head_dim, int group) { return group * head_dim > 512 ? 16 : 24; }
 constexpr int kPlanThreads = 1024;  // both planning kernels run one workgroup of this size
 
 // One item = a contiguous page range of one request.  Read by a wave with one
@@ -107,6 +125,7 @@ struct PlanParams {
   const int32_t* indices;
   const int32_t* last_page_len;
   int batch, hkv, target_units, max_items;
+  int direct;  // splits merged in one level at most (direct_splits)
   DecodeHeader* header;
   DecodeItem* items;
   int* counters;
@@ -287,6 +306,11 @@ __device__ inline void write_item(const PlanParams& p, int idx, const int* scan,
     for (int j = 0; j < kInlinePages; ++j) it.pages[j] = -1;
   }
   p.items[first + sp] = it;
+  // the group counters of a request merged in two levels (the merge counters
+  // of all of them are zeroed by the callers)
+  const int groups = split_groups(nsr, p.direct);
+  if (groups > 1 && sp < groups)
+    for (int h = 0; h < p.hkv; ++h) p.counters[((base + r) * p.hkv + h) * kCounterStride + 1 + sp] = 0;
 }
 
 __device__ inline void write_header(const PlanParams& p, int running, int q16) {

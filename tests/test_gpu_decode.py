@@ -368,3 +368,31 @@ def test_repeated_runs_are_bit_identical(dev, parity, hq, hkv, d, lo, hi):
     for o in outs[1:]:
         assert torch.equal(o, outs[0])
     parity(outs[0].float().cpu(), _ref(b))
+
+
+# (heads, context): one request; head_dim 128 merges up to 24 splits in one
+# level with groups of up to 4 Q heads and 16 with more, head_dim 64 24, 256 by
+# how many 16-byte loads its heads take
+@pytest.mark.parametrize("hq,hkv,d,ctx,nsplit", [
+    (32, 8, 128, 16 * 64 - 3, 16), (32, 8, 128, 16 * 96, 24), (32, 8, 128, 16 * 97 + 5, 25),  # the last direct one
+    (28, 4, 128, 16 * 64, 16), (28, 4, 128, 16 * 65, 17), (64, 8, 128, 16 * 256 - 15, 59),  # (the other requests take their part of the units)
+    (8, 1, 128, 16 * 257, 65), (5, 1, 128, 16 * 1024 - 1, 256), (6, 1, 128, 16 * 1028 + 1, 258),  # groups of 16, of 24
+    (14, 2, 64, 16 * 100, 25), (4, 1, 64, 32768, 505), (2, 2, 64, 16 * 260, 65),
+    (16, 4, 256, 16 * 65, 17), (4, 2, 256, 16 * 100, 25), (8, 1, 256, 16 * 900, 225),
+])
+def test_splits_merged_in_two_levels(dev, parity, hq, hkv, d, ctx, nsplit):
+    """Either side of each group count of the two-level merge, between requests
+    that merge directly and one that is not split; the same bits on every run of
+    a plan (the merge and group counters are back at zero), and over a workspace
+    that held other bytes before."""
+    b = make_paged_batch([17, ctx, 200, 5], hq, hkv, d, seed=ctx + d)
+    pool, q, ip, ix, lp = to_dev(b, dev)
+    w = _wrapper(dev)
+    w._ws.fill_(0x5b)
+    w.plan(ip, ix, lp, hq, hkv, d, 16)
+    items = w._ws[256:256 + 128 * 600].view(torch.int32).view(-1, 32).cpu()
+    of_request = items[(items[:, 24] == 1) & (items[:, 29] > 0) & (items[:, 29] < 1 << 16)]
+    assert int(of_request[0, 29]) == nsplit
+    outs = [w.run(q, pool).cpu() for _ in range(3)]
+    parity(outs[0].float(), _ref(b))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
