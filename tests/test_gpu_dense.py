@@ -181,3 +181,18 @@ def test_few_row_linear_routes(dev):
     with pytest.raises(ValueError):
         from minimal_inference_amd import _lib
         _lib.call("mi_linear", x.data_ptr(), 512, w.data_ptr(), None, b.data_ptr(), 256, 33, 256, 512, 0)
+
+
+def test_silu_mul_every_gate(dev):
+    """Every bf16 gate (zeros, subnormals, infinities, NaNs and those whose
+    exponential is past the end of fp32) times one: the bits of the fp32 formula
+    with an IEEE division; and more rows than the grid's second axis has."""
+    from minimal_inference_amd.dense import silu_mul
+
+    gate = torch.arange(-32768, 32768, device=dev, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    out = silu_mul(torch.cat([gate, torch.ones_like(gate)])[None])[0]
+    ref = (gate.float() / (1 + torch.exp(-gate.float()))).to(torch.bfloat16)
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert torch.equal(out.nan_to_num(7.0).view(torch.int16), ref.nan_to_num(7.0).view(torch.int16))
+    gu = torch.randn(65535 + 70, 48, device=dev, generator=torch.Generator(device=dev).manual_seed(3)).to(torch.bfloat16)
+    assert _ulp_close(silu_mul(gu), F.silu(gu[:, :24]) * gu[:, 24:], 1)
