@@ -362,6 +362,12 @@ int mi_silu_mul(const void* gate_up, int64_t gate_up_stride, void* out, int64_t 
 int mi_linear(const void* x, int64_t x_stride, const void* weight, const void* bias, void* out,
               int64_t out_stride, int32_t rows, int32_t n, int32_t k, mi_stream_t stream);
 
+/* mi_linear_silu: mi_silu_mul of mi_linear's result (no bias) in one launch, the
+ * same bits: weight [2 n][k] holds the n gate rows, then the n up rows; out
+ * [rows][n] = silu(gate) * up (MLP, model.py:301-311). */
+int mi_linear_silu(const void* x, int64_t x_stride, const void* weight, void* out, int64_t out_stride,
+                   int32_t rows, int32_t n, int32_t k, mi_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

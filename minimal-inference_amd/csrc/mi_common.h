@@ -51,6 +51,29 @@ __device__ __forceinline__ uint16_t cvt_bf16(float f) { return uint16_t(cvt_pk_b
 // rounded to bf16 anyway.
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
+// g / (1 + exp(-g)) in fp32.  The quotient is the hardware reciprocal's with one
+// Newton step and one residual step, which rounds as the IEEE division does (the
+// reciprocal alone is 1 ulp off often enough to turn a bf16 rounding, and the
+// product with u would double that); the fix-up returns zeros, infinities and
+// NaN.  Below -80 the denominator is scaled, so that the reciprocal of one near
+// the end of the range does not flush to zero.
+__device__ __forceinline__ float silu(float g) {
+  const float d = 1.0f + expf(-g);
+  const float s = g < -80.f ? 0x1p-24f : 1.0f;
+  const float e = d * s;
+  float r = fast_rcp(e);
+  r = fmaf(fmaf(-e, r, 1.0f), r, r);
+  float q = g * r;
+  q = fmaf(fmaf(-e, q, g), r, q);
+  return __builtin_amdgcn_div_fixupf(q * s, d, g);
+}
+
+// bf16(bf16(silu(g)) * u) of two bf16 pairs
+__device__ __forceinline__ uint32_t silu_mul_bf16x2(uint32_t g, uint32_t u) {
+  const uint32_t a = cvt_pk_bf16(silu(bf16_lo(g)), silu(bf16_hi(g)));
+  return cvt_pk_bf16(bf16_lo(a) * bf16_lo(u), bf16_hi(a) * bf16_hi(u));
+}
+
 // ---------------------------------------------------------------- MFMA types
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;

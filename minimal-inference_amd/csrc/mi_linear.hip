@@ -39,7 +39,7 @@ struct LinearParams {
   const uint16_t* bias;  // null: none
   uint16_t* out;
   int64_t o_stride;
-  int rows, n, k;
+  int rows, n, k;  // n: columns of out
 };
 
 __device__ __forceinline__ u32x4_t lds_load16(const lds_t* p) {
@@ -59,20 +59,27 @@ struct LinearTraits {
   static_assert(SMEM <= 160 * 1024, "LDS");
 };
 
-template <int R, int MB, int D>
+// GLU: W holds n gate rows, then n up rows; tile r is the gate's (even r) or the
+// up part's (odd) of the output columns 16 (r / 2) .., and out = silu(gate) * up,
+// rounded where the separate kernel rounds.  It saves that launch (of eight rows'
+// 3.5 us) and the write and read of gate and up.
+template <int R, int MB, int D, bool GLU>
 __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
+  constexpr int HALVES = GLU ? 2 : 1, COLS = 16 * R / HALVES;  // output columns of a workgroup
+  static_assert(R % HALVES == 0, "gate and up tiles in pairs");
   using T = LinearTraits<R, MB, D>;
   __shared__ __attribute__((aligned(16))) char smem[T::SMEM];
   lds_t* const lds = (lds_t*)smem;
   const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int g = lane >> 4, n = lane & 15;
-  const int row0 = int(blockIdx.x) * 16 * R;
+  const int row0 = int(blockIdx.x) * COLS;
   const int nslab = p.k / kSlab, steps = (nslab - w + kWaves - 1) / kWaves;  // this wave's: w, w + 4, ...
 
   // load i of a slab: 8 rows, lane l chunk l % 8 of row l / 8; rows past the
   // end read out of range: zeros
   const char* wbase = reinterpret_cast<const char*>(p.w) + int64_t(row0) * p.k * 2;
-  const int wsize = min(16 * R, p.n - row0) * p.k * 2;
+  const int wsize = min(COLS, p.n - row0) * p.k * 2;  // of each half
+  const int64_t up = int64_t(p.n) * p.k * 2;
   const int xsize = int(((p.rows - 1) * p.x_stride + p.k) * 2);
   const int lr = lane / 8, lc = (lane % 8) * 16;
   const int wv = lr * p.k * 2 + lc, wrow8 = 8 * p.k * 2;
@@ -81,13 +88,18 @@ __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
   auto load = [&](int d, int step) {
     const int off = (step * kWaves + w) * kSlabBytes;
     const bool ok = step < steps;
-    const __amdgpu_buffer_rsrc_t rw =
-        __builtin_amdgcn_make_buffer_rsrc((void*)(wbase + off), (short)0, ok ? wsize - off : 0, kBufferWord3);
+    __amdgpu_buffer_rsrc_t rw[HALVES];
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+      rw[h] = __builtin_amdgcn_make_buffer_rsrc((void*)(wbase + h * up + off), (short)0, ok ? wsize - off : 0,
+                                                kBufferWord3);
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(reinterpret_cast<const char*>(p.x) + off), (short)0, ok ? xsize - off : 0, kBufferWord3);
     // W is read once: non-temporal
 #pragma unroll
-    for (int i = 0; i < 2 * R; ++i) wr[d][i] = __builtin_amdgcn_raw_buffer_load_b128(rw, wv + i * wrow8, 0, kCacheNT);
+    for (int i = 0; i < 2 * R; ++i)
+      wr[d][i] = __builtin_amdgcn_raw_buffer_load_b128(
+          rw[(i / 2) % HALVES], wv + (i / 2 / HALVES * 2 + i % 2) * wrow8, 0, kCacheNT);
 #pragma unroll
     for (int i = 0; i < 2 * MB; ++i) xr[d][i] = __builtin_amdgcn_raw_buffer_load_b128(rx, xv + i * xrow8, 0, 0);
   };
@@ -150,12 +162,16 @@ __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
     for (int b = 0; b < MB; ++b)
       lds_store16(lds + (w * R * MB + r * MB + b) * 1024 + lane * 16, __builtin_bit_cast(u32x4_t, acc[r][b]));
   __syncthreads();
-  for (int q = w; q < R * MB; q += kWaves) {
-    const int r = q / MB, b = q - r * MB;
+  auto total = [&](int q) {
     mi::f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int o = 0; o < kWaves; ++o)
       sum += __builtin_bit_cast(mi::f32x4_t, lds_load16(lds + (o * R * MB + q) * 1024 + lane * 16));
+    return sum;
+  };
+  for (int q = w; q < R / HALVES * MB; q += kWaves) {
+    const int r = q / MB, b = q - r * MB;  // r: the tile (or pair of tiles)
+    mi::f32x4_t sum = total(HALVES * r * MB + b);
     const int m = b * 16 + n, col = row0 + r * 16 + 4 * g;
     if (m < p.rows && row0 + r * 16 < p.n) {
       if (p.bias) {
@@ -165,8 +181,13 @@ __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
         sum[2] += mi::bf16_lo(bb.y);
         sum[3] += mi::bf16_hi(bb.y);
       }
-      *reinterpret_cast<u32x2_t*>(p.out + int64_t(m) * p.o_stride + col) =
-          u32x2_t{mi::cvt_pk_bf16(sum[0], sum[1]), mi::cvt_pk_bf16(sum[2], sum[3])};
+      u32x2_t v = {mi::cvt_pk_bf16(sum[0], sum[1]), mi::cvt_pk_bf16(sum[2], sum[3])};
+      if constexpr (GLU) {
+        const mi::f32x4_t u = total((HALVES * r + 1) * MB + b);
+        v[0] = mi::silu_mul_bf16x2(v[0], mi::cvt_pk_bf16(u[0], u[1]));
+        v[1] = mi::silu_mul_bf16x2(v[1], mi::cvt_pk_bf16(u[2], u[3]));
+      }
+      *reinterpret_cast<u32x2_t*>(p.out + int64_t(m) * p.o_stride + col) = v;
     }
   }
 }
@@ -189,8 +210,8 @@ typedef void (*LinearKernel)(LinearParams);
 // workgroup bound it (D 4, as for long K); two tiles when the launch is so long
 // that starting and ending workgroups shows.  With two blocks of x, what bounds
 // it is x from L2, so as many tiles as still leave workgroups for the CUs.
-template <int R, int D>
-LinearKernel pick(int mb) { return mb == 1 ? linear_kernel<R, 1, D> : linear_kernel<R, 2, D>; }
+template <int R, int D, bool GLU = false>
+LinearKernel pick(int mb) { return mb == 1 ? linear_kernel<R, 1, D, GLU> : linear_kernel<R, 2, D, GLU>; }
 
 LinearKernel pick_kernel(int tiles, int k, int mb, int* r) {
   if (mb == 1) {
@@ -201,21 +222,37 @@ LinearKernel pick_kernel(int tiles, int k, int mb, int* r) {
   return *r == 1 ? pick<1, 2>(2) : *r == 2 ? pick<2, 2>(2) : pick<4, 2>(2);
 }
 
-}  // namespace
+// With the gated product, from the pairs of a gate and an up tile (us at 8 / 32
+// rows; separate = the forms above and the SiLU kernel after them):
+//                      pairs       R 2          R 4       separate
+//   N  9728 K   896      304    6.6 /  8.1   5.9 /  6.9   8.6 /  9.2
+//   N  9728 K  4096      304   19.4 / 23.3  19.4 / 20.2  20.4 / 22.3
+//   N 19456 K  2048      608   16.5 / 20.1  20.2 / 22.5  20.4 / 24.9
+//   N 28672 K  4096      896   39.2 / 47.8  42.6 / 43.6  41.1 / 46.8
+//   N 37888 K  3584     1184   43.5 / 53.9  46.9 / 52.0  44.9 / 55.5
+// Two pairs where that costs no CU more tiles (fewer reads of x): of a launch of
+// one round, and with two blocks of x of any.  (D 4 is slower on all but 59,136 x
+// 8,192, where it is equal.)
+LinearKernel pick_glu(int pairs, int mb, int* r) {
+  const bool two = ((pairs + 1) / 2 + 255) / 256 * 2 <= (pairs + 255) / 256;
+  *r = two && (mb == 2 || pairs <= 512) ? 4 : 2;
+  return *r == 4 ? pick<4, 2, true>(mb) : pick<2, 2, true>(mb);
+}
 
-extern "C" int mi_linear(const void* x, int64_t x_stride, const void* weight, const void* bias, void* out,
-                         int64_t out_stride, int32_t rows, int32_t n, int32_t k, mi_stream_t stream) {
+// Both entry points; `halves` 2: gate and up rows, n output columns.
+int launch_linear(const char* name, const void* x, int64_t x_stride, const void* weight, const void* bias, void* out,
+                  int64_t out_stride, int32_t rows, int32_t n, int32_t k, int halves, mi_stream_t stream) {
   mi::clear_error();
   if (rows < 0 || rows > kMaxRows || n <= 0 || n % 16 || k <= 0 || k % kSlab || k > (1 << 24))
-    return mi::fail(MI_ERR_INVALID, "linear: rows %d (0..%d), n %d (multiple of 16), k %d (multiple of %d)", rows,
-                    kMaxRows, n, k, kSlab);
+    return mi::fail(MI_ERR_INVALID, "%s: rows %d (0..%d), n %d (multiple of 16), k %d (multiple of %d)", name,
+                    rows, kMaxRows, n, k, kSlab);
   if (rows == 0) return MI_OK;
-  if (!x || !weight || !out) return mi::fail(MI_ERR_INVALID, "linear: null pointer argument");
+  if (!x || !weight || !out) return mi::fail(MI_ERR_INVALID, "%s: null pointer argument", name);
   if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(weight) & 15) ||
       (reinterpret_cast<uintptr_t>(bias) & 7) || (reinterpret_cast<uintptr_t>(out) & 7) || x_stride % 8 || out_stride % 4)
-    return mi::fail(MI_ERR_INVALID, "linear: x rows and weight must be 16-byte, bias and out rows 8-byte aligned");
+    return mi::fail(MI_ERR_INVALID, "%s: x rows and weight must be 16-byte, bias and out rows 8-byte aligned", name);
   if (x_stride < k || out_stride < n || int64_t(rows) * x_stride > (1 << 29))
-    return mi::fail(MI_ERR_INVALID, "linear: row strides %lld / %lld for k %d, n %d", (long long)x_stride,
+    return mi::fail(MI_ERR_INVALID, "%s: row strides %lld / %lld for k %d, n %d", name, (long long)x_stride,
                     (long long)out_stride, k, n);
   LinearParams p;
   p.x = static_cast<const uint16_t*>(x);
@@ -229,7 +266,20 @@ extern "C" int mi_linear(const void* x, int64_t x_stride, const void* weight, co
   p.k = k;
   const int mb = (rows + 15) / 16;
   int r = 1;
-  const LinearKernel kernel = pick_kernel(n / 16, k, mb, &r);
-  hipLaunchKernelGGL(kernel, dim3((n / 16 + r - 1) / r), dim3(64 * kWaves), 0, static_cast<hipStream_t>(stream), p);
+  const LinearKernel kernel = halves == 2 ? pick_glu(n / 16, mb, &r) : pick_kernel(n / 16, k, mb, &r);
+  const int per = r / halves;  // output tiles of a workgroup
+  hipLaunchKernelGGL(kernel, dim3((n / 16 + per - 1) / per), dim3(64 * kWaves), 0, static_cast<hipStream_t>(stream), p);
   return mi::check_launch("linear_kernel");
+}
+
+}  // namespace
+
+extern "C" int mi_linear(const void* x, int64_t x_stride, const void* weight, const void* bias, void* out,
+                         int64_t out_stride, int32_t rows, int32_t n, int32_t k, mi_stream_t stream) {
+  return launch_linear("linear", x, x_stride, weight, bias, out, out_stride, rows, n, k, 1, stream);
+}
+
+extern "C" int mi_linear_silu(const void* x, int64_t x_stride, const void* weight, void* out, int64_t out_stride,
+                              int32_t rows, int32_t n, int32_t k, mi_stream_t stream) {
+  return launch_linear("linear_silu", x, x_stride, weight, nullptr, out, out_stride, rows, n, k, 2, stream);
 }

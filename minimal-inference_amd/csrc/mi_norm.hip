@@ -115,23 +115,6 @@ struct SiluMulParams {
   int64_t rows;
 };
 
-// g / (1 + exp(-g)) in fp32.  The quotient is the hardware reciprocal's with one
-// Newton step and one residual step, which rounds as the IEEE division does (the
-// reciprocal alone is 1 ulp off often enough to turn a bf16 rounding, and the
-// product with u would double that); the fix-up returns zeros, infinities and
-// NaN.  Below -80 the denominator is scaled, so that the reciprocal of one near
-// the end of the range does not flush to zero.
-__device__ __forceinline__ float silu(float g) {
-  const float d = 1.0f + expf(-g);
-  const float s = g < -80.f ? 0x1p-24f : 1.0f;
-  const float e = d * s;
-  float r = mi::fast_rcp(e);
-  r = fmaf(fmaf(-e, r, 1.0f), r, r);
-  float q = g * r;
-  q = fmaf(fmaf(-e, q, g), r, q);
-  return __builtin_amdgcn_div_fixupf(q * s, d, g);
-}
-
 // One thread per 8 outputs (16 bytes of g, of u and of out) of a row; the grid's
 // second axis walks the rows.  Bound: HBM.  With the scaled division, the software
 // roundings and an index division per thread it was VALU bound: 18,240 x 14,336
@@ -147,10 +130,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(SiluMulParams p) {
     const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
     uint32_t ow[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t a = mi::cvt_pk_bf16(silu(mi::bf16_lo(gw[k])), silu(mi::bf16_hi(gw[k])));
-      ow[k] = mi::cvt_pk_bf16(mi::bf16_lo(a) * mi::bf16_lo(uw[k]), mi::bf16_hi(a) * mi::bf16_hi(uw[k]));
-    }
+    for (int k = 0; k < 4; ++k) ow[k] = mi::silu_mul_bf16x2(gw[k], uw[k]);
     st16(p.out + row * p.o_stride + ch * 8, make_uint4(ow[0], ow[1], ow[2], ow[3]));
   }
 }

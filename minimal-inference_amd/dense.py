@@ -6,7 +6,9 @@ model.py:324-344; RMSNorm, model.py:115-122); ``silu_mul(gate_up)`` for
 ``F.silu(gate) * up`` over the fused gate/up projection (MLP,
 model.py:301-311).  Both run one HIP kernel (``mi_add_rms_norm`` /
 ``mi_silu_mul``); there is no torch fallback.  ``linear(x, weight, bias)`` is
-``F.linear`` with a decode step's few rows on ``mi_linear``.
+``F.linear`` with a decode step's few rows on ``mi_linear``, and
+``linear_silu(x, gate_up)`` is ``silu_mul(linear(x, gate_up))`` with those rows
+in one launch (``mi_linear_silu``).
 """
 
 from __future__ import annotations
@@ -86,22 +88,43 @@ def _few_rows(rows: int, n: int, k: int) -> bool:
     return rows <= LINEAR_MAX_ROWS and k < 8192
 
 
+def _takes(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
+    """Whether ``linear`` runs on the few-row kernel."""
+    rows, k = x.shape
+    n = weight.shape[0]
+    return not (rows == 0 or not _few_rows(rows, n, k) or n % 16 or k % 64 or not x.is_cuda
+                or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device
+                or weight.shape[1] != k or not weight.is_contiguous() or x.stride(1) != 1 or x.stride(0) % 8
+                or x.stride(0) < k or x.data_ptr() % 16 or weight.data_ptr() % 16
+                or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
+                or (bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (n,)
+                                          or not bias.is_contiguous() or bias.device != x.device
+                                          or bias.data_ptr() % 8
+                                          or (torch.is_grad_enabled() and bias.requires_grad))))
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``F.linear`` of [rows, k]; a decode step's few rows of bf16 go to the kernel
     that streams the weight once (fp32 accumulation, one rounding), everything else
     to torch."""
+    if not _takes(x, weight, bias):
+        return F.linear(x, weight, bias)
     rows, k = x.shape
     n = weight.shape[0]
-    if (rows == 0 or not _few_rows(rows, n, k) or n % 16 or k % 64 or not x.is_cuda
-            or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device
-            or weight.shape[1] != k or not weight.is_contiguous() or x.stride(1) != 1 or x.stride(0) % 8
-            or x.stride(0) < k or x.data_ptr() % 16 or weight.data_ptr() % 16
-            or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
-            or (bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (n,) or not bias.is_contiguous()
-                                      or bias.device != x.device or bias.data_ptr() % 8
-                                      or (torch.is_grad_enabled() and bias.requires_grad)))):
-        return F.linear(x, weight, bias)
     out = torch.empty(rows, n, dtype=x.dtype, device=x.device)
     _lib.call("mi_linear", x.data_ptr(), x.stride(0), weight.data_ptr(), bias.data_ptr() if bias is not None else None,
               out.data_ptr(), n, rows, n, k, stream_of(x))
+    return out
+
+
+def linear_silu(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
+    """``silu_mul(linear(x, gate_up))``, the same bits, in one launch where ``linear``
+    runs on the few-row kernel."""
+    rows, k = x.shape
+    n = gate_up.shape[0] // 2
+    if n % 16 or gate_up.shape[0] % 2 or not _takes(x, gate_up, None):
+        return silu_mul(linear(x, gate_up))
+    out = torch.empty(rows, n, dtype=x.dtype, device=x.device)
+    _lib.call("mi_linear_silu", x.data_ptr(), x.stride(0), gate_up.data_ptr(), out.data_ptr(), n, rows, n, k,
+              stream_of(x))
     return out

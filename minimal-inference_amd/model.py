@@ -18,11 +18,12 @@ does both itself (``run_rope_append``; ``fused_decode=False`` keeps the
 separate launch), bit-identical again; ``fused_rope=False`` keeps the
 separate ops.
 By default the residual adds and the RMSNorms that follow them run as one
-HIP kernel each, and SiLU(gate) * up as one (``dense.add_rms_norm`` /
-``dense.silu_mul``, fp32 math, one bf16 rounding per output), and the
-projections of a decode step's few rows on the kernel that streams each weight
-once (``dense.linear``); ``fused_dense=False`` keeps torch's ``F.linear``,
-``F.rms_norm``, adds and ``F.silu(g) * u``.  RoPE tables are held in the model dtype, as the reference's are after ``.to(dtype)``
+HIP kernel each (``dense.add_rms_norm``, fp32 math, one bf16 rounding per
+output), the projections of a decode step's few rows on the kernel that streams
+each weight once (``dense.linear``), SiLU(gate) * up in that launch too or, for
+more rows, as a kernel of its own (``dense.linear_silu``);
+``fused_dense=False`` keeps torch's ``F.linear``, ``F.rms_norm``, adds and
+``F.silu(g) * u``.  RoPE tables are held in the model dtype, as the reference's are after ``.to(dtype)``
 (server.py:251).  Weights are random-initialised on the device (N(0, 0.02),
 norms 1) -- the benchmark configurations use random weights.
 """
@@ -37,7 +38,7 @@ import os
 import torch
 import torch.nn.functional as F
 
-from .dense import add_rms_norm, linear, silu_mul
+from .dense import add_rms_norm, linear, linear_silu
 from .page import append_paged_kv_cache, rope_append_paged_kv_cache
 
 
@@ -243,7 +244,7 @@ class Model:
                 continue
             # x += o W_o; h = rms(x); x += down(silu(g) * u); h = next layer's rms(x)
             h = add_rms_norm(x, project(o.view(t, nq * d), L.w_o), L.post_norm, eps)
-            down = project(silu_mul(project(h, L.w_gate_up)), L.w_down)
+            down = project(linear_silu(h, L.w_gate_up), L.w_down)
             if li + 1 < len(self.layers):
                 h = add_rms_norm(x, down, self.layers[li + 1].in_norm, eps)
             elif last_rows is None:

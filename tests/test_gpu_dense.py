@@ -196,3 +196,42 @@ def test_silu_mul_every_gate(dev):
     assert torch.equal(out.nan_to_num(7.0).view(torch.int16), ref.nan_to_num(7.0).view(torch.int16))
     gu = torch.randn(65535 + 70, 48, device=dev, generator=torch.Generator(device=dev).manual_seed(3)).to(torch.bfloat16)
     assert _ulp_close(silu_mul(gu), F.silu(gu[:, :24]) * gu[:, 24:], 1)
+
+
+@pytest.mark.parametrize("inter,k", [(16, 64), (48, 896), (4096, 128), (4112, 64), (4864, 896), (8208, 64), (14336, 256)])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32])
+def test_few_row_linear_silu(dev, rows, inter, k):
+    """mi_linear_silu at the edges of its forms (one and two blocks of rows, one
+    and two pairs of tiles to a workgroup, a last workgroup half empty): the bits
+    of the two separate kernels; nothing written around the rows."""
+    from minimal_inference_amd import _lib
+    from minimal_inference_amd.dense import silu_mul
+
+    g = torch.Generator(device=dev).manual_seed(rows * 131 + inter + k)
+    big = torch.randn(rows, k + 64, device=dev, generator=g).to(torch.bfloat16)
+    x = big[:, 32:32 + k]
+    w = torch.randn(2 * inter, k, device=dev, generator=g).to(torch.bfloat16)
+    gu = torch.empty(rows, 2 * inter, device=dev, dtype=torch.bfloat16)
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.call("mi_linear", x.data_ptr(), x.stride(0), w.data_ptr(), None, gu.data_ptr(), 2 * inter, rows, 2 * inter, k,
+              stream)
+    out = torch.full((rows + 1, inter + 8), 7.0, device=dev, dtype=torch.bfloat16)
+    _lib.call("mi_linear_silu", x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), out.stride(0), rows, inter, k,
+              stream)
+    assert torch.equal(out[:rows, :inter], silu_mul(gu))
+    assert bool((out[rows] == 7.0).all()) and bool((out[:, inter:] == 7.0).all())
+
+
+def test_few_row_linear_silu_routes(dev):
+    """dense.linear_silu is silu_mul(linear(..)), bit for bit, where the one launch
+    takes the call and where it does not (more rows, narrow halves, strided
+    weights), and refuses what silu_mul refuses."""
+    from minimal_inference_amd.dense import linear, linear_silu, silu_mul
+
+    x = torch.randn(8, 512, device=dev).to(torch.bfloat16)
+    w = torch.randn(256, 512, device=dev).to(torch.bfloat16)
+    for xx, ww in [(x, w), (x.repeat(5, 1), w), (x, w[:240]), (x[:, :480], w[:, :480]), (x[:0], w)]:
+        assert torch.equal(linear_silu(xx, ww), silu_mul(linear(xx, ww)))
+    for xx, ww in [(x, w[:255]), (x.float(), w.float())]:
+        with pytest.raises((ValueError, TypeError)):
+            linear_silu(xx, ww)
