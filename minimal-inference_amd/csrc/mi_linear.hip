@@ -63,10 +63,16 @@ struct LinearTraits {
 // up part's (odd) of the output columns 16 (r / 2) .., and out = silu(gate) * up,
 // rounded where the separate kernel rounds.  It saves that launch (of eight rows'
 // 3.5 us) and the write and read of gate and up.
-template <int R, int MB, int D, bool GLU>
+//
+// HALF: only the first 8 rows of the one tile, for weights of so few rows that
+// most CUs had no workgroup.  The matrix instructions' other 8 rows hold what is
+// in LDS and are not written out.
+template <int R, int MB, int D, bool GLU, bool HALF>
 __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
-  constexpr int HALVES = GLU ? 2 : 1, COLS = 16 * R / HALVES;  // output columns of a workgroup
+  constexpr int HALVES = GLU ? 2 : 1, COLS = HALF ? 8 : 16 * R / HALVES;  // output columns of a workgroup
   static_assert(R % HALVES == 0, "gate and up tiles in pairs");
+  static_assert(!HALF || (R == 1 && !GLU), "half of one tile");
+  constexpr int WL = HALF ? 1 : 2 * R;  // loads of 8 rows of W per slab
   using T = LinearTraits<R, MB, D>;
   __shared__ __attribute__((aligned(16))) char smem[T::SMEM];
   lds_t* const lds = (lds_t*)smem;
@@ -84,7 +90,7 @@ __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
   const int lr = lane / 8, lc = (lane % 8) * 16;
   const int wv = lr * p.k * 2 + lc, wrow8 = 8 * p.k * 2;
   const int xv = int(lr * p.x_stride * 2) + lc, xrow8 = int(8 * p.x_stride * 2);
-  u32x4_t wr[D][2 * R], xr[D][2 * MB];
+  u32x4_t wr[D][WL], xr[D][2 * MB];
   auto load = [&](int d, int step) {
     const int off = (step * kWaves + w) * kSlabBytes;
     const bool ok = step < steps;
@@ -97,7 +103,7 @@ __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
         (void*)(reinterpret_cast<const char*>(p.x) + off), (short)0, ok ? xsize - off : 0, kBufferWord3);
     // W is read once: non-temporal
 #pragma unroll
-    for (int i = 0; i < 2 * R; ++i)
+    for (int i = 0; i < WL; ++i)
       wr[d][i] = __builtin_amdgcn_raw_buffer_load_b128(
           rw[(i / 2) % HALVES], wv + (i / 2 / HALVES * 2 + i % 2) * wrow8, 0, kCacheNT);
 #pragma unroll
@@ -130,7 +136,7 @@ __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
 #pragma unroll
-      for (int i = 0; i < 2 * R; ++i) lds_store16(slot + i * 1024 + so[i & 1], wr[d][i]);
+      for (int i = 0; i < WL; ++i) lds_store16(slot + i * 1024 + so[i & 1], wr[d][i]);
 #pragma unroll
       for (int i = 0; i < 2 * MB; ++i) lds_store16(slot + (2 * R + i) * 1024 + so[i & 1], xr[d][i]);
       load(d, s0 + d + D);
@@ -173,7 +179,7 @@ __global__ __launch_bounds__(64 * kWaves) void linear_kernel(LinearParams p) {
     const int r = q / MB, b = q - r * MB;  // r: the tile (or pair of tiles)
     mi::f32x4_t sum = total(HALVES * r * MB + b);
     const int m = b * 16 + n, col = row0 + r * 16 + 4 * g;
-    if (m < p.rows && row0 + r * 16 < p.n) {
+    if (m < p.rows && row0 + r * 16 < p.n && (!HALF || g < 2)) {
       if (p.bias) {
         const u32x2_t bb = *reinterpret_cast<const u32x2_t*>(p.bias + col);
         sum[0] += mi::bf16_lo(bb.x);
@@ -210,16 +216,24 @@ typedef void (*LinearKernel)(LinearParams);
 // workgroup bound it (D 4, as for long K); two tiles when the launch is so long
 // that starting and ending workgroups shows.  With two blocks of x, what bounds
 // it is x from L2, so as many tiles as still leave workgroups for the CUs.
-template <int R, int D, bool GLU = false>
-LinearKernel pick(int mb) { return mb == 1 ? linear_kernel<R, 1, D, GLU> : linear_kernel<R, 2, D, GLU>; }
+// Half tiles up to 128 tiles (full ones leave half of the CUs or more idle), with
+// two blocks of x, which they read twice as often, for long k only (us at 8 / 32 rows,
+// whole / half): 896 x 4,864 6.8 / 10.3, 5.6 / 9.2; 2,048 x 8,960 11.4 / 18.1, 9.1 / 15.7;
+// 1,024 x 3,072 5.1 / 7.4, 4.3 / 6.7; 1,536 x 1,536 4.1 / 5.0, 3.8 / 5.3; 896 x 896
+// 3.2 / 4.0, 3.05 / 4.0.  (8 waves, or D 8, with either: slower.)
+template <int R, int D, bool GLU = false, bool HALF = false>
+LinearKernel pick(int mb) { return mb == 1 ? linear_kernel<R, 1, D, GLU, HALF> : linear_kernel<R, 2, D, GLU, HALF>; }
 
-LinearKernel pick_kernel(int tiles, int k, int mb, int* r) {
-  if (mb == 1) {
-    *r = tiles > 2048 ? 2 : 1;
-    return *r == 2 ? pick<2, 2>(1) : tiles <= 256 || k >= 8192 ? pick<1, 4>(1) : pick<1, 2>(1);
+LinearKernel pick_kernel(int tiles, int k, int mb, int* cols) {
+  if (tiles <= 128 && (mb == 1 || k >= 2048)) {
+    *cols = 8;
+    return pick<1, 4, false, true>(mb);
   }
-  *r = tiles <= 256 ? 1 : tiles < 512 ? 2 : 4;
-  return *r == 1 ? pick<1, 2>(2) : *r == 2 ? pick<2, 2>(2) : pick<4, 2>(2);
+  const int r = mb == 1 ? (tiles > 2048 ? 2 : 1) : tiles <= 256 ? 1 : tiles < 512 ? 2 : 4;
+  *cols = 16 * r;
+  if (mb == 1 && (r == 2 || (tiles > 256 && k < 8192))) return r == 2 ? pick<2, 2>(1) : pick<1, 2>(1);
+  if (mb == 1) return linear_kernel<1, 1, 4, false, false>;
+  return r == 1 ? pick<1, 2>(2) : r == 2 ? pick<2, 2>(2) : pick<4, 2>(2);
 }
 
 // With the gated product, from the pairs of a gate and an up tile (us at 8 / 32
@@ -233,10 +247,11 @@ LinearKernel pick_kernel(int tiles, int k, int mb, int* r) {
 // Two pairs where that costs no CU more tiles (fewer reads of x): of a launch of
 // one round, and with two blocks of x of any.  (D 4 is slower on all but 59,136 x
 // 8,192, where it is equal.)
-LinearKernel pick_glu(int pairs, int mb, int* r) {
-  const bool two = ((pairs + 1) / 2 + 255) / 256 * 2 <= (pairs + 255) / 256;
-  *r = two && (mb == 2 || pairs <= 512) ? 4 : 2;
-  return *r == 4 ? pick<4, 2, true>(mb) : pick<2, 2, true>(mb);
+LinearKernel pick_glu(int pairs, int mb, int* cols) {
+  const bool even = ((pairs + 1) / 2 + 255) / 256 * 2 <= (pairs + 255) / 256;
+  const bool two = even && (mb == 2 || pairs <= 512);
+  *cols = two ? 32 : 16;
+  return two ? pick<4, 2, true>(mb) : pick<2, 2, true>(mb);
 }
 
 // Both entry points; `halves` 2: gate and up rows, n output columns.
@@ -265,10 +280,9 @@ int launch_linear(const char* name, const void* x, int64_t x_stride, const void*
   p.n = n;
   p.k = k;
   const int mb = (rows + 15) / 16;
-  int r = 1;
-  const LinearKernel kernel = halves == 2 ? pick_glu(n / 16, mb, &r) : pick_kernel(n / 16, k, mb, &r);
-  const int per = r / halves;  // output tiles of a workgroup
-  hipLaunchKernelGGL(kernel, dim3((n / 16 + per - 1) / per), dim3(64 * kWaves), 0, static_cast<hipStream_t>(stream), p);
+  int cols = 16;  // output columns of a workgroup
+  const LinearKernel kernel = halves == 2 ? pick_glu(n / 16, mb, &cols) : pick_kernel(n / 16, k, mb, &cols);
+  hipLaunchKernelGGL(kernel, dim3((n + cols - 1) / cols), dim3(64 * kWaves), 0, static_cast<hipStream_t>(stream), p);
   return mi::check_launch("linear_kernel");
 }
 

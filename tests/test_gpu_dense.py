@@ -130,6 +130,7 @@ def test_model_prefill_logits_fused_vs_unfused(dev):
     (4112, 4096), (8176, 128), (8208, 576),                       # either side of 256 and 512 tiles of 16 columns
     (32768, 256), (32800, 256), (151936, 896),                    # 2,048 tiles, past them with a partial last workgroup
     (512, 8192), (16, 18944),                                     # long rows
+    (2048, 1984), (2048, 2048), (2064, 2048),                     # either side of half tiles
 ])
 def test_few_row_linear(dev, rows, n, k):
     """mi_linear at the edges of its forms against an fp32 product of the same
