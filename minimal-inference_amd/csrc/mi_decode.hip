@@ -319,8 +319,12 @@ __device__ __forceinline__ void publish_merge(const RunParams& p, int u, int b, 
   };
   // this unit's group: splits first .. first + n1 - 1
   const int groups = split_groups(nsplit, direct_splits(D, G));
-  const int grp = groups == 1 ? 0 : ((u / p.hkv - item_base + 1) * groups - 1) / nsplit;
-  const int first = grp * nsplit / groups, n1 = (grp + 1) * nsplit / groups - first;
+  int grp = 0, first = 0, n1 = nsplit;  // (the divisions stay off the path of one level)
+  if (groups > 1) {
+    grp = ((u / p.hkv - item_base + 1) * groups - 1) / nsplit;
+    first = grp * nsplit / groups;
+    n1 = (grp + 1) * nsplit / groups - first;
+  }
   int* const my_counter = counter + (groups == 1 ? 0 : 1 + grp);
   if (count(my_counter) != n1 - 1) return;
 
