@@ -6,14 +6,15 @@ import torch
 
 
 def stream_of(t: torch.Tensor) -> int:
-    """Raw hipStream_t of torch's current stream on ``t``'s device."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Raw hipStream_t of torch's current stream on ``t``'s device (the handle itself:
+    a ``Stream`` object around it cost each call 1.9 us, this 0.1)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def require_gpu(name: str, t: torch.Tensor) -> None:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be on a GPU (got {t.device}); there is no CPU path")
 
 
