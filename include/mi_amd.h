@@ -199,9 +199,16 @@ int mi_decode_static(const void* q, int64_t q_stride_batch, int64_t q_stride_hea
  * head, and the query positions per workgroup depend on both.
  * A workspace larger than mi_prefill_workspace_size also holds partial
  * results at its end (never more than three quarters of it): launches of few
- * rows over many keys are then cut along the keys and merged.  128 MiB is
- * enough for every shape; a smaller one only splits less, with the same
- * results within rounding.
+ * rows over many keys are then cut into finer units, also along the keys, and
+ * merged.  128 MiB is enough for every shape; a smaller one only splits less,
+ * with the same results within rounding.  The partials belong to one run at a
+ * time, so a run uses them only on the stream its plan was made on, outside of
+ * graph capture, and with the plan's workspace (address and size) and head
+ * counts.  Every other run -- on other streams, in a graph, of a copy of the
+ * workspace's first mi_prefill_workspace_size bytes -- takes whole tiles and
+ * only reads the workspace: runs of one plan may overlap, as any that only read.
+ * (A run never outlives its stream: a handle that is destroyed and made again
+ * counts as the same stream.)
  * head_dim in {64, 128, 256}; page_size == 16.
  * ------------------------------------------------------------------------ */
 size_t mi_prefill_workspace_size(int32_t batch_size, int64_t total_q);

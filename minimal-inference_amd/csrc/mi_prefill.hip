@@ -18,10 +18,13 @@
 // that leave most of the chip idle take fine tiles of one row block per wave
 // instead, and tiles with long key ranges are cut into units along the keys
 // whose fp32 partials the last unit merges (prefill_plan_kernel says when and
-// why).  plan() lists the units request
+// why).  plan() lists the tiles, and where it pays the units, request
 // by request (longest prompt first), each request's tiles heaviest first; the
-// grid maps unit-major, so the XCD that a KV head's workgroups land on runs
-// one request's tiles back to back and finds its K / V in L2.
+// grid maps them tile-major, so the XCD that a KV head's workgroups land on runs
+// one request's tiles back to back and finds its K / V in L2.  The units'
+// partials lie in the workspace, so only runs in the order of the plan's stream
+// use them; every other run takes the tiles and only reads the workspace
+// (RunKey).
 //
 // Per 64-key tile: the workgroup stages K and V in LDS (double buffered: the
 // next tile's global loads are in flight while this one is consumed; one
@@ -39,6 +42,7 @@
 #include <math.h>
 
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "mi_common.h"
@@ -89,15 +93,33 @@ struct alignas(32) PrefillTile {
 };
 constexpr unsigned kToEnd = 0xffffu;
 
-struct PrefillHeader {
-  int num_tiles;
-  int error;
-  int bm;             // query positions per tile
-  int row_blocks;     // 16-row blocks per wave: the coarse or the fine form of the tiles
-  int chunk;          // KV tiles per unit at most (0: no tile is split)
-  int slots;          // partial slots per KV head (the counters follow them)
-  int64_t split_off;  // byte offset of the partial slots in the workspace
+// Which runs may take the units of a plan: the partials and their counters
+// belong to one run at a time, and nothing but the order of a stream says that
+// two runs do not overlap.  So a run takes the units only on the stream the plan
+// was made on, with the plan's workspace (address and size: a copy of a
+// workspace has no partials of its own) and geometry, and outside of graph
+// capture (a graph's replays are ordered with nothing else); the plan's
+// `serial`, in the header and in front of the units, tells a header that was put
+// back over a later plan's units.  Every other run takes the tile list, which
+// needs the workspace's first mi_prefill_workspace_size bytes only and writes
+// none of them.
+struct RunKey {
+  uint64_t ws, bytes, stream, shape;
 };
+
+struct PrefillHeader {
+  int num_tiles;   // whole coarse tiles, behind the header
+  int error;
+  int bm;          // query positions per tile of the units
+  int row_blocks;  // their 16-row blocks per wave: the coarse or the fine form
+  int chunk;       // KV tiles per unit at most (0: no tile is split)
+  int slots;       // partial slots per KV head (the counters follow them)
+  int units;       // 0: every run takes the tiles
+  int pad;
+  RunKey key;
+  uint64_t serial;
+};
+static_assert(sizeof(PrefillHeader) <= 256, "the tiles start at byte 256");
 
 // Waves per workgroup.
 constexpr int waves_for(int /*head_dim*/) { return 4; }
@@ -153,25 +175,49 @@ constexpr size_t partial_bytes(int head_dim, int blocks) {
 constexpr int kCounterStride = 32;  // ints: one 128-byte line per merge counter
 constexpr int kMaxSplits = 64;      // per tile
 
-// Partial slots per KV head of coarse and of fine units and their offset: the
-// end of the workspace, at most three quarters of it and two resident rounds
-// of coarse units.  No slots when the workspace is too small to be worth
-// splitting for: the plan then splits nothing.
-struct PartialLayout {
-  size_t off;
-  int coarse, fine;
+// The units and their partials: the end of the workspace, at most three
+// quarters of it and two resident rounds of coarse units.  At `off` the serial
+// of the plan whose units these are, 256 bytes further the units (room for
+// kFineRounds resident rounds), at `parts` the partial slots (per KV head
+// `coarse` of coarse or `fine` of fine units) and behind them the counters.  No
+// slots when the workspace is too small to be worth it: the plan then makes
+// tiles only.
+struct UnitLayout {
+  size_t off, parts;
+  int capacity, coarse, fine;
 };
-PartialLayout partial_layout(size_t workspace_bytes, int hkv, int head_dim) {
+UnitLayout unit_layout(size_t workspace_bytes, int hkv, int head_dim) {
   const auto per = [&](int blocks) { return (partial_bytes(head_dim, blocks) + kCounterStride * sizeof(int)) * size_t(hkv); };
-  PartialLayout L{0, 0, 0};
-  const size_t c = std::min(workspace_bytes / 4 * 3 / per(row_blocks(head_dim)),
-                            size_t(2 * resident_groups(head_dim) / hkv));
-  const size_t bytes = c * per(row_blocks(head_dim)) + 256;
-  if (c < 2 || bytes + 256 + sizeof(PrefillTile) > workspace_bytes) return L;
-  L.off = (workspace_bytes - c * per(row_blocks(head_dim))) & ~size_t(255);
+  UnitLayout L{0, 0, 0, 0, 0};
+  const size_t coarse = per(row_blocks(head_dim)), limit = workspace_bytes / 4 * 3;
+  const int capacity = kFineRounds * resident_groups(head_dim) / hkv;
+  const size_t list = 256 + mi::align_up(size_t(capacity) * sizeof(PrefillTile), 256);
+  const size_t c = limit < list ? 0 : std::min((limit - list) / coarse, size_t(2 * resident_groups(head_dim) / hkv));
+  if (c < 2 || list + c * coarse + 512 + sizeof(PrefillTile) > workspace_bytes) return L;
+  L.off = (workspace_bytes - c * coarse - list) & ~size_t(255);
+  L.parts = L.off + list;
+  L.capacity = capacity;
   L.coarse = int(c);
-  L.fine = int(std::min(c * per(row_blocks(head_dim)) / per(1), size_t(0xffff)));
+  L.fine = int(std::min(c * coarse / per(1), size_t(0xffff)));
   return L;
+}
+
+// The stream that orders the calls made on `s`, as RunKey has it: 0 for none
+// (under capture the launch happens in replays on any stream; the per-thread
+// default stream is one handle for many streams).
+uint64_t ordering_stream(hipStream_t s) {
+  if (s == hipStreamPerThread) return 0;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return status == hipStreamCaptureStatusNone ? reinterpret_cast<uint64_t>(s) + 1 : 0;
+}
+
+RunKey run_key(const void* ws, size_t bytes, int hkv, int group, int head_dim, hipStream_t s) {
+  return RunKey{reinterpret_cast<uint64_t>(ws), bytes, ordering_stream(s),
+                uint64_t(unsigned(hkv)) << 32 | uint64_t(unsigned(group)) << 16 | uint64_t(unsigned(head_dim) & 0xffff)};
 }
 
 struct PlanParams {
@@ -184,11 +230,15 @@ struct PlanParams {
   int bm[2], blocks[2], slots[2];  // positions, row blocks per wave and partial slots of fine [0] and coarse [1] tiles
   size_t counters_off[2];          // of the merge counters, behind the partials
   int resident;                    // workgroups resident at once
-  int split_capacity;              // units the list holds in front of the partial slots
-  int64_t split_off;
+  int tile_room;                   // tiles the list holds in front of the units
+  int unit_capacity;               // 0: tiles only
   char* ws;
   PrefillHeader* header;
   PrefillTile* tiles;
+  PrefillTile* units;
+  uint64_t* unit_serial;
+  RunKey key;
+  uint64_t serial;
 };
 
 constexpr int kPlanThreads = 1024;
@@ -235,19 +285,23 @@ __device__ __forceinline__ PrefillTile make_tile(int bm, int qo, int kv, int q0,
   return tile;
 }
 
-__device__ __forceinline__ void write_header(const PlanParams& p, int form, int units, int ntiles, int chunk) {
-  p.header->num_tiles = units;
+// `ntiles` coarse tiles, `fit` of them listed
+__device__ __forceinline__ void write_header(const PlanParams& p, int ntiles, int fit, int form, int units, int chunk) {
+  p.header->num_tiles = fit;
   p.header->error = ntiles > p.capacity ? 1 : 0;
   p.header->bm = p.bm[form];
   p.header->row_blocks = p.blocks[form];
   p.header->chunk = chunk;
   p.header->slots = p.slots[form];
-  p.header->split_off = p.split_off;
+  p.header->units = units;
+  p.header->key = p.key;
+  p.header->serial = p.serial;
+  if (units > 0) *p.unit_serial = p.serial;
 }
 
 // Batches of more requests than the block has threads: one request per thread
 // and round, its place found by counting the requests ordered before it in
-// global memory; coarse tiles, none of them split.
+// global memory; tiles only.
 __device__ void plan_large(const PlanParams& p, int* wsum) {
   const int t = threadIdx.x, bm = p.bm[1];
   int total = 0;
@@ -269,7 +323,7 @@ __device__ void plan_large(const PlanParams& p, int* wsum) {
     block_scan(nt, wsum, &chunk_total);
     total += chunk_total;
   }
-  if (t == 0) write_header(p, 1, min(total, p.capacity), total, 0);
+  if (t == 0) write_header(p, total, min(total, p.capacity), 1, 0, 0);
 }
 
 // Tile order: requests by decreasing prompt length (ties by index), each
@@ -292,7 +346,8 @@ __device__ void plan_large(const PlanParams& p, int* wsum) {
 // 160 -> 168 us: the partials of three row blocks are 104 KB per unit).  The
 // count assumes a causal run; the last
 // unit of a tile takes whatever keys remain, so a non-causal run of the same
-// plan is complete too.
+// plan is complete too.  The whole coarse tiles are listed in any case, for the
+// runs that may not take the units (RunKey).
 __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p) {
   __shared__ int s_qo[kPlanThreads], s_kv[kPlanThreads], s_q0[kPlanThreads], s_pb0[kPlanThreads];
   __shared__ int s_req[kPlanThreads], s_end[kPlanThreads], wsum[kPlanThreads / 64];
@@ -335,11 +390,6 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
     area += __int_as_float(red[0][i]);
     fine_tiles += __int_as_float(red[1][i]);
   }
-  // fine or coarse tiles (see kFineLoad)
-  const float fine_load = area * float(p.group * p.hkv) / (64.f * kKvTile * float(p.resident));
-  const int form = p.blocks[1] > 1 && fine_load <= float(kFineLoad) &&
-                           fine_tiles * float(p.hkv) <= float(kFineRounds * p.resident) ? 0 : 1;
-  const int bm = p.bm[form], nslots = p.slots[form];
   int rank = 0;
   for (int c = 0; c < p.batch; ++c) {
     const int qc = s_qo[c];
@@ -347,15 +397,20 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
   }
   if (t < p.batch) {
     s_req[rank] = t;
-    s_end[rank] = (qo + bm - 1) / bm;
   }
   __syncthreads();
-  int ntiles = 0;
-  const int end = block_scan(t < p.batch ? s_end[t] : 0, wsum, &ntiles);
-  s_end[t] = end;
-  if (t < p.batch && end <= p.capacity) atomicMax(&s_fit, end);
-  __syncthreads();
-  const int fit = s_fit;  // tiles of the requests that fit the list
+  // tiles up to the end of each request, in rank order
+  int bm = p.bm[1];
+  auto scan_tiles = [&]() {
+    int total = 0;
+    const int end = block_scan(t < p.batch ? (s_qo[s_req[t]] + bm - 1) / bm : 0, wsum, &total);
+    s_end[t] = end;
+    if (t < p.batch && end <= p.capacity) atomicMax(&s_fit, end);
+    __syncthreads();
+    return total;
+  };
+  int ntiles = scan_tiles();
+  const int coarse_tiles = ntiles, fit = s_fit;  // fit: tiles of the requests that fit the list
 
   // tile i of the list: its request's rank, and its causal KV tiles
   auto rank_of = [&](int i) {
@@ -374,10 +429,22 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
   auto kv_tiles = [&](const PrefillTile& x) {
     return (max(0, min(x.kv_len, x.row0 + x.q_rows + x.kv_len - x.qo_len)) + kKvTile - 1) / kKvTile;
   };
+  for (int i = t; i < fit; i += kPlanThreads) p.tiles[i] = tile_of(i);
+  // fine or coarse units (see kFineLoad)
+  const bool room = p.unit_capacity > 0 && ntiles == fit && fit <= p.tile_room;
+  const float fine_load = area * float(p.group * p.hkv) / (64.f * kKvTile * float(p.resident));
+  const int form = room && p.blocks[1] > 1 && fine_load <= float(kFineLoad) &&
+                           fine_tiles * float(p.hkv) <= float(kFineRounds * p.resident) ? 0 : 1;
+  const int nslots = p.slots[form];
+  if (form == 0) {
+    __syncthreads();  // s_end's readers are done
+    bm = p.bm[0];
+    ntiles = scan_tiles();
+  }
   // the units that fill the rounds which the unsplit tiles need
   const int rounds = (ntiles * p.hkv + p.resident - 1) / p.resident;
-  const int limit = min(rounds * p.resident / p.hkv, p.split_capacity);
-  const bool consider = nslots > 0 && (form == 0 || rounds == 1) && ntiles == fit && ntiles <= min(kSplitTiles, limit);
+  const int limit = min(rounds * p.resident / p.hkv, p.unit_capacity);
+  const bool consider = room && (form == 0 || rounds == 1) && ntiles <= min(kSplitTiles, limit);
   int chunk = 0, longest = 0;
   if (consider) {
     int sum = 0;
@@ -434,9 +501,10 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
       chunk = lo < longest ? lo : 0;
     }
   }
-  int units = fit;
+  // whole fine tiles are units, whole coarse ones the tiles that are listed already
+  int units = form == 0 && ntiles <= p.unit_capacity ? ntiles : 0;
   if (chunk == 0) {
-    for (int i = t; i < fit; i += kPlanThreads) p.tiles[i] = tile_of(i);
+    for (int i = t; i < units; i += kPlanThreads) p.units[i] = tile_of(i);
   } else {
     // units in tile order; the scan carries the units and, above them, the
     // partial slots before each tile
@@ -456,7 +524,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
           const unsigned kb = unsigned(s * n / ns), ke = s + 1 < ns ? unsigned((s + 1) * n / ns) : kToEnd;
           x.kt = int(kb | ke << 16);
           x.part = ns > 1 ? ((slot0 + s) << 16 | s << 8 | ns) : 0;
-          p.tiles[u0 + s] = x;
+          p.units[u0 + s] = x;
         }
       }
       units += all & 0xffff;
@@ -466,13 +534,17 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
     int* counters = reinterpret_cast<int*>(p.ws + p.counters_off[form]);
     for (int i = t; i < slots * p.hkv; i += kPlanThreads) counters[i * kCounterStride] = 0;
   }
-  if (t == 0) write_header(p, form, units, ntiles, chunk);
+  if (t == 0) write_header(p, coarse_tiles, fit, form, units, chunk);
 }
 
 struct RunParams {
-  char* ws;
   const PrefillHeader* header;
   const PrefillTile* tiles;
+  const PrefillTile* units;       // (any address where there is no room for them)
+  const uint64_t* unit_serial;
+  char* parts;
+  RunKey key;
+  int tile_bm;                    // positions per coarse tile
   const uint16_t* q;
   int64_t q_st, q_sh;
   int64_t q_ext;  // elements one position's heads span: (heads - 1) * q_sh + head_dim
@@ -589,9 +661,9 @@ __device__ __forceinline__ void stage_rows(lds_t* ob, int r, int lane, const mi:
                        mi::cvt_pk_bf16(o[j][2] * inv[2], o[j][3] * inv[3])});
 }
 
-// Where the plan keeps the partials (PrefillHeader).
+// Where the partials are, and how many slots there are per KV head.
 struct PartialArea {
-  int64_t off;
+  char* base;
   int slots;
 };
 
@@ -616,7 +688,7 @@ __device__ __forceinline__ bool merge_splits(const RunParams& p, int part, const
   static_assert(WB * T::WAVES == int(partial_bytes(D, MAXRB)), "partial layout");
   const int g = lane >> 4;
   const int nsplit = part & 0xff, split = (part >> 8) & 0xff, slot0 = int(unsigned(part) >> 16) - split;
-  char* base = p.ws + pa.off;
+  char* base = pa.base;
   const int nslots = pa.slots;
   // the wave's partial of split s, one descriptor each: the slots of one tile
   // and KV head lie hkv slots apart
@@ -1113,8 +1185,8 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
   }
 }
 
-// The plan says which form its tiles have: coarse, RB row blocks per wave, or
-// fine, one.
+// The units of the plan if this run may take them, else its tiles.  The plan
+// says which form the units have: coarse, RB row blocks per wave, or fine, one.
 template <int D, int RB>
 __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void prefill_run_kernel(RunParams p) {
   __shared__ __attribute__((aligned(16))) char smem[PrefillTraits<D, RB>::SMEM];  // [buffer][K, V], then the output rows
@@ -1130,12 +1202,20 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
   typedef __attribute__((address_space(4))) const PrefillHeader const_header;
   typedef __attribute__((address_space(4))) const int const_int;
   const const_header* h = (const const_header*)(p.header);
-  if (tile_idx >= h->num_tiles) return;  // whole workgroup
-  const const_int* f = (const const_int*)(p.tiles + tile_idx);
+  typedef __attribute__((address_space(4))) const uint64_t const_u64;
+  // (without branches: the compiler then loads all of it in one round trip; one
+  // test after the other cost a run 0.7 us)
+  const uint64_t serial = *(const const_u64*)(p.unit_serial);
+  const int num_units = h->units, num_tiles = h->num_tiles, unit_bm = h->bm, blocks = h->row_blocks;
+  const uint64_t differs = (h->key.ws ^ p.key.ws) | (h->key.bytes ^ p.key.bytes) | (h->key.stream ^ p.key.stream) |
+                           (h->key.shape ^ p.key.shape) | (h->serial ^ serial) | uint64_t(p.key.stream == 0);
+  const PartialArea pa{p.parts, h->slots};
+  const bool own = (num_units > 0) & (differs == 0) & (int64_t(num_units) * p.hkv <= int64_t(gridDim.x));
+  if (tile_idx >= (own ? num_units : num_tiles)) return;  // whole workgroup
+  const const_int* f = (const const_int*)((own ? p.units : p.tiles) + tile_idx);
   const PrefillTile t{f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
-  const PartialArea pa{h->split_off, h->slots};
-  const int bm = h->bm;
-  if (RB > 1 && h->row_blocks == 1) run_unit<D, 1>(p, t, pa, hkv, bm, lds);
+  const int bm = own ? unit_bm : p.tile_bm;
+  if (RB > 1 && own && blocks == 1) run_unit<D, 1>(p, t, pa, hkv, bm, lds);
   else run_unit<D, RB>(p, t, pa, hkv, bm, lds);
 }
 
@@ -1173,18 +1253,23 @@ extern "C" int mi_prefill_plan(void* workspace, size_t workspace_bytes, const in
   pp.group = num_qo_heads / num_kv_heads;
   pp.hkv = num_kv_heads;
   pp.resident = resident_groups(head_dim);
-  const PartialLayout L = partial_layout(workspace_bytes, num_kv_heads, head_dim);
-  pp.split_off = int64_t(L.off);
-  pp.split_capacity = L.coarse ? int(std::min<size_t>((L.off - 256) / sizeof(PrefillTile), 1 << 30)) : 0;
+  const UnitLayout L = unit_layout(workspace_bytes, num_kv_heads, head_dim);
+  static std::atomic<uint64_t> plans{0};
+  pp.serial = (plans.fetch_add(1, std::memory_order_relaxed) + 1) * 0x9e3779b97f4a7c15ull;
+  pp.key = run_key(workspace, workspace_bytes, num_kv_heads, pp.group, head_dim, static_cast<hipStream_t>(stream));
+  pp.unit_capacity = pp.key.stream ? L.capacity : 0;
+  pp.tile_room = L.capacity ? int(std::min<size_t>((L.off - 256) / sizeof(PrefillTile), 1 << 30)) : 0;
   for (int form = 0; form < 2; ++form) {
     pp.blocks[form] = form ? row_blocks(head_dim) : 1;
     pp.bm[form] = rows_per_tile(pp.group, head_dim, pp.blocks[form]);
     pp.slots[form] = form ? L.coarse : L.fine;
-    pp.counters_off[form] = L.off + size_t(pp.slots[form]) * num_kv_heads * partial_bytes(head_dim, pp.blocks[form]);
+    pp.counters_off[form] = L.parts + size_t(pp.slots[form]) * num_kv_heads * partial_bytes(head_dim, pp.blocks[form]);
   }
   pp.ws = ws;
   pp.header = reinterpret_cast<PrefillHeader*>(ws);
   pp.tiles = reinterpret_cast<PrefillTile*>(ws + 256);
+  pp.unit_serial = reinterpret_cast<uint64_t*>(ws + L.off);
+  pp.units = reinterpret_cast<PrefillTile*>(ws + L.off + 256);
   hipLaunchKernelGGL(prefill_plan_kernel, dim3(1), dim3(kPlanThreads), 0, static_cast<hipStream_t>(stream), pp);
   return mi::check_launch("prefill_plan_kernel");
 }
@@ -1219,9 +1304,14 @@ extern "C" int mi_prefill_run(void* workspace, size_t workspace_bytes, const voi
   if (grid > 0x7fffffff) return mi::fail(MI_ERR_INVALID, "prefill run: too many tiles");
   char* ws = static_cast<char*>(workspace);
   RunParams rp;
-  rp.ws = ws;
   rp.header = reinterpret_cast<const PrefillHeader*>(ws);
   rp.tiles = reinterpret_cast<const PrefillTile*>(ws + 256);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const UnitLayout L = unit_layout(workspace_bytes, num_kv_heads, head_dim);
+  rp.unit_serial = reinterpret_cast<const uint64_t*>(ws + L.off);
+  rp.units = reinterpret_cast<const PrefillTile*>(ws + L.off + 256);
+  rp.parts = ws + L.parts;
+  rp.key = run_key(workspace, workspace_bytes, num_kv_heads, num_qo_heads / num_kv_heads, head_dim, s);
   rp.q = static_cast<const uint16_t*>(q);
   rp.q_st = q_stride_token;
   rp.q_sh = q_stride_head;
@@ -1235,7 +1325,7 @@ extern "C" int mi_prefill_run(void* workspace, size_t workspace_bytes, const voi
   rp.hkv = num_kv_heads;
   rp.group = num_qo_heads / num_kv_heads;
   rp.causal = causal ? 1 : 0;
-  const int bm = rows_per_tile(rp.group, head_dim, row_blocks(head_dim));
+  const int bm = rp.tile_bm = rows_per_tile(rp.group, head_dim, row_blocks(head_dim));
   // a tile addresses its q / out rows through one buffer descriptor each, by
   // 32-bit byte offsets from its first position: any strides (heads inside a
   // position's row, or head-major) whose tile extent fits
@@ -1249,7 +1339,6 @@ extern "C" int mi_prefill_run(void* workspace, size_t workspace_bytes, const voi
   const float scale = sm_scale > 0.f ? sm_scale : 1.0f / sqrtf(float(head_dim));
   rp.scale_log2 = scale * mi::kLog2e;
   const dim3 g{static_cast<uint32_t>(grid), 1u, 1u};
-  hipStream_t s = static_cast<hipStream_t>(stream);
   switch (head_dim) {
     case 64: hipLaunchKernelGGL((prefill_run_kernel<64, 2>), g, dim3(64 * waves_for(64)), 0, s, rp); break;
     case 128: hipLaunchKernelGGL((prefill_run_kernel<128, 3>), g, dim3(64 * waves_for(128)), 0, s, rp); break;

@@ -11,6 +11,11 @@ Reference usage:
 of requests can share one call (``qo_indptr`` with B+1 entries); the
 reference only ever passes one, and prefills requests one after another.
 Any integer GQA group runs without Q-head padding.
+
+Runs of one plan may overlap.  Those on the stream that ``plan`` was called on
+(outside of graph capture) may cut the keys into units whose partials the
+workspace holds; the others take whole tiles and only read the workspace, with
+the same results within rounding.
 """
 
 from __future__ import annotations

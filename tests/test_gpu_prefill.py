@@ -280,3 +280,120 @@ def test_tiles_split_over_the_keys(dev, parity, heads, qo_lens, cached, blocks, 
     header, whole = run(int(_lib.load().mi_prefill_workspace_size(len(qo_lens), total)))
     assert header[1] == 0 and header[4] == 0
     parity(whole[0].float(), ref)
+
+
+class _Planned:
+    """A batch on the GPU, and what runs of its plan give that take whole tiles
+    (a workspace of the least size) and that take the units."""
+
+    def __init__(self, dev, heads, qo_lens, cached, seed):
+        from minimal_inference_amd import _lib
+
+        self.dev, self.heads, self.total = dev, heads, sum(qo_lens)
+        hq, hkv, d = heads
+        b = make_paged_batch([q + c for q, c in zip(qo_lens, cached)], hq, hkv, d, seed=seed)
+        qo = [0]
+        for n in qo_lens:
+            qo.append(qo[-1] + n)
+        self.batch = len(qo_lens)
+        self.csr = [torch.tensor(qo, dtype=torch.int32, device=dev), torch.tensor(b["indptr"], dtype=torch.int32, device=dev),
+                    b["indices"].to(dev), torch.tensor(b["last"], dtype=torch.int32, device=dev)]
+        self.pool = b["pool"].to(dev)
+        g = torch.Generator(device=dev).manual_seed(seed)
+        self.q = [torch.randn(self.total, hq, d, device=dev, generator=g).to(torch.bfloat16) for _ in range(3)]
+        self.need = int(_lib.load().mi_prefill_workspace_size(self.batch, self.total))
+        self.w, self.ws = self.plan(128 << 20)
+        self.units = [self.w.run(q, self.pool) for q in self.q]
+        small, _ = self.plan(self.need)
+        self.whole = [small.run(q, self.pool) for q in self.q]
+        torch.cuda.synchronize()
+
+    def plan(self, nbytes, ws=None):
+        from minimal_inference_amd.prefill import BatchPrefillWithPagedKVCacheWrapper
+
+        ws = torch.full((nbytes,), 0x5a, dtype=torch.uint8, device=self.dev) if ws is None else ws
+        w = BatchPrefillWithPagedKVCacheWrapper(ws, "NHD")
+        w.plan(*self.csr, *self.heads, 16, causal=True, max_total_q=self.total)
+        return w, ws
+
+    def run_abi(self, ws, q, pool, heads):
+        """mi_prefill_run of whatever plan `ws` holds."""
+        from minimal_inference_amd import _lib
+
+        out = torch.empty_like(q)
+        _lib.call("mi_prefill_run", ws.data_ptr(), ws.numel(), q.data_ptr(), q.stride(0), q.stride(1), pool.data_ptr(),
+                  pool.shape[0], self.csr[2].data_ptr(), out.data_ptr(), out.stride(0), out.stride(1), self.batch,
+                  self.total, *heads, 16, 1, 0.0, torch.cuda.current_stream().cuda_stream)
+        return out
+
+
+OWNED_CASES = [((32, 8, 128), [3], [1000]), ((64, 8, 128), [200, 37], [5001, 3000]), ((14, 2, 64), [700], [4010]),
+               ((16, 4, 256), [70], [2500])]
+
+
+@pytest.mark.parametrize("heads,qo_lens,cached", OWNED_CASES)
+def test_runs_outside_of_the_plans_stream_only_read_the_workspace(dev, heads, qo_lens, cached):
+    """Runs of one plan that nothing orders: those on other streams than the
+    plan's and those of a graph take whole tiles and leave every byte of the
+    workspace alone, so they may overlap each other and one on the plan's
+    stream."""
+    c = _Planned(dev, heads, qo_lens, cached, seed=31)
+    assert not torch.equal(c.units[0], c.whole[0])  # (split rows round differently)
+    before = c.ws.clone()
+    torch.cuda.synchronize()
+    sides = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for s in sides:
+        with torch.cuda.stream(s):
+            out = c.w.run(c.q[0], c.pool)
+        s.synchronize()
+        assert torch.equal(out, c.whole[0])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = c.w.run(c.q[1], c.pool)
+    for _ in range(3):
+        captured.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, c.whole[1]) and torch.equal(c.ws, before)
+        assert torch.equal(c.w.run(c.q[1], c.pool), c.units[1])
+        before = c.ws.clone()
+    # all of them at once
+    outs = []
+    for i in range(12):
+        outs.append((c.w.run(c.q[i % 3], c.pool), c.units[i % 3]))
+        for k, s in enumerate(sides):
+            with torch.cuda.stream(s):
+                outs.append((c.w.run(c.q[(i + k) % 3], c.pool), c.whole[(i + k) % 3]))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in outs)
+
+
+@pytest.mark.parametrize("heads,qo_lens,cached", OWNED_CASES)
+def test_saved_plans_and_other_geometry_take_whole_tiles(dev, heads, qo_lens, cached):
+    """A plan's bytes in another buffer (whole, or the documented least size), put
+    back over a later plan's, or run with other head counts of the same group:
+    the partials belong to the plan in place, so these runs take whole tiles and
+    write nothing but the output."""
+    c = _Planned(dev, heads, qo_lens, cached, seed=32)
+    saved = c.ws[:c.need].clone()
+    for copy in (c.ws.clone(), saved.clone()):
+        kept = copy.clone()
+        assert torch.equal(c.run_abi(copy, c.q[0], c.pool, heads), c.whole[0])
+        assert torch.equal(copy, kept)
+    assert torch.equal(c.run_abi(c.ws, c.q[0], c.pool, heads), c.units[0])  # (in place)
+    other = _Planned(dev, heads, [n + 5 for n in qo_lens], cached, seed=33)
+    other.plan(0, ws=c.ws)
+    c.ws[:c.need].copy_(saved)
+    kept = c.ws.clone()
+    assert torch.equal(c.run_abi(c.ws, c.q[0], c.pool, heads), c.whole[0])
+    assert torch.equal(c.ws, kept)
+    # twice the heads, in groups of the same size
+    hq, hkv, d = heads
+    q2, pool2 = torch.cat([c.q[0], c.q[1]], 1), torch.cat([c.pool, c.pool.flip(0)], 3)
+    c.plan(0, ws=c.ws)
+    kept = c.ws.clone()
+    out2 = c.run_abi(c.ws, q2, pool2, (2 * hq, 2 * hkv, d))
+    assert torch.equal(out2[:, :hq], c.whole[0])
+    flipped, _ = c.plan(c.need)
+    assert torch.equal(out2[:, hq:], flipped.run(c.q[1], pool2[:, :, :, hkv:].contiguous()))
+    assert torch.equal(c.ws, kept)
