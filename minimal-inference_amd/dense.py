@@ -74,8 +74,10 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Te
     return out
 
 
-# Most rows the few-row kernel takes.
+# What the few-row kernel takes at most: rows, elements that x's rows span, k.
 LINEAR_MAX_ROWS = 32
+LINEAR_MAX_SPAN = 1 << 29
+LINEAR_MAX_K = 1 << 23
 
 
 def _few_rows(rows: int, n: int, k: int) -> bool:
@@ -92,10 +94,11 @@ def _takes(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> 
     """Whether ``linear`` runs on the few-row kernel."""
     rows, k = x.shape
     n = weight.shape[0]
-    return not (rows == 0 or not _few_rows(rows, n, k) or n % 16 or k % 64 or not x.is_cuda
+    return not (weight.dim() != 2 or rows == 0 or n == 0 or not 0 < k <= LINEAR_MAX_K
+                or not _few_rows(rows, n, k) or n % 16 or k % 64 or not x.is_cuda
                 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device
                 or weight.shape[1] != k or not weight.is_contiguous() or x.stride(1) != 1 or x.stride(0) % 8
-                or x.stride(0) < k or x.data_ptr() % 16 or weight.data_ptr() % 16
+                or x.stride(0) < k or rows * x.stride(0) > LINEAR_MAX_SPAN or x.data_ptr() % 16 or weight.data_ptr() % 16
                 or (torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad))
                 or (bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (n,)
                                           or not bias.is_contiguous() or bias.device != x.device

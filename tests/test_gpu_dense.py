@@ -236,3 +236,22 @@ def test_few_row_linear_silu_routes(dev):
     for xx, ww in [(x, w[:255]), (x.float(), w.float())]:
         with pytest.raises((ValueError, TypeError)):
             linear_silu(xx, ww)
+
+
+def test_few_row_linear_leaves_what_the_kernel_refuses_to_torch(dev):
+    """Rows whose stride spans more than mi_linear's 2^29 elements, and weights of
+    no rows, no columns or one axis, are F.linear's."""
+    from minimal_inference_amd.dense import linear, linear_silu, silu_mul
+
+    step, k = (1 << 28) + 8, 512
+    far = torch.zeros(step + k, device=dev, dtype=torch.bfloat16)
+    x = far.as_strided((2, k), (step, 1))
+    x.copy_(torch.randn(2, k, device=dev))
+    w = torch.randn(256, k, device=dev).to(torch.bfloat16)
+    assert torch.equal(linear(x, w), F.linear(x, w))
+    assert torch.equal(linear_silu(x, w), silu_mul(F.linear(x, w)))
+    near = x.contiguous()
+    assert torch.equal(linear(near, w[:0]), F.linear(near, w[:0]))
+    assert torch.equal(linear(near, w[0]), F.linear(near, w[0]))
+    for ww in (w[:, :0], torch.empty(256, 0, device=dev, dtype=torch.bfloat16)):
+        assert torch.equal(linear(near[:, :0], ww), torch.zeros(2, 256, device=dev, dtype=torch.bfloat16))
