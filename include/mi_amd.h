@@ -364,7 +364,7 @@ int mi_silu_mul(const void* gate_up, int64_t gate_up_stride, void* out, int64_t 
  * MLP and LM head: model.py:160-163, 245-252, 301-311, 432-435), fp32
  * accumulation, one rounding.  x [rows][k] and out [rows][n] with the given
  * row strides (elements), weight [n][k] contiguous, bias [n] or null; rows
- * 0..32, n a multiple of 16, k of 64; x rows and weight 16-byte, bias and out
+ * 0..32, n a multiple of 16, k of 64 and at most 2^23; x rows and weight 16-byte, bias and out
  * rows 8-byte aligned.  No workspace; the result does not depend on timing. */
 int mi_linear(const void* x, int64_t x_stride, const void* weight, const void* bias, void* out,
               int64_t out_stride, int32_t rows, int32_t n, int32_t k, mi_stream_t stream);

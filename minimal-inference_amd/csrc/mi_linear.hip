@@ -24,6 +24,7 @@ constexpr int kWaves = 4;
 constexpr int kSlab = 64;             // k per slab
 constexpr int kSlabBytes = kSlab * 2;  // of one row
 constexpr int kMaxRows = 32;
+constexpr int kMaxK = 1 << 23;  // the byte size of a workgroup's rows of W (up to 64) is an int
 constexpr int kBufferWord3 = 0x00020000;
 // Cache-policy operand of the buffer intrinsics: nt (non-temporal / streaming).
 constexpr int kCacheNT = 2;
@@ -258,9 +259,9 @@ LinearKernel pick_glu(int pairs, int mb, int* cols) {
 int launch_linear(const char* name, const void* x, int64_t x_stride, const void* weight, const void* bias, void* out,
                   int64_t out_stride, int32_t rows, int32_t n, int32_t k, int halves, mi_stream_t stream) {
   mi::clear_error();
-  if (rows < 0 || rows > kMaxRows || n <= 0 || n % 16 || k <= 0 || k % kSlab || k > (1 << 24))
-    return mi::fail(MI_ERR_INVALID, "%s: rows %d (0..%d), n %d (multiple of 16), k %d (multiple of %d)", name,
-                    rows, kMaxRows, n, k, kSlab);
+  if (rows < 0 || rows > kMaxRows || n <= 0 || n % 16 || k <= 0 || k % kSlab || k > kMaxK)
+    return mi::fail(MI_ERR_INVALID, "%s: rows %d (0..%d), n %d (multiple of 16), k %d (multiple of %d, at most %d)", name,
+                    rows, kMaxRows, n, k, kSlab, kMaxK);
   if (rows == 0) return MI_OK;
   if (!x || !weight || !out) return mi::fail(MI_ERR_INVALID, "%s: null pointer argument", name);
   if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(weight) & 15) ||

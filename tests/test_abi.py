@@ -89,3 +89,8 @@ def test_host_only_calls_and_error_reporting():
     assert "16-byte aligned" in _lib.last_error()
     assert prefill_rc(q_sh=1 << 26) == _lib.MI_ERR_INVALID
     assert "2^30" in _lib.last_error()
+    # few-row linear: a workgroup's 64 rows of W must span less than 2^31 bytes
+    for rows in (32, 1):
+        rc = lib.mi_linear(fake, 1 << 24, fake, None, fake, 16, rows, 16, 1 << 24, None)
+        assert rc == _lib.MI_ERR_INVALID
+        assert f"at most {1 << 23}" in _lib.last_error()
