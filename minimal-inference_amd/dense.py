@@ -15,6 +15,10 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+from torch._C import _len_torch_dispatch_stack
+from torch._C._functorch import peek_interpreter_stack
+from torch.autograd import forward_ad
+from torch.overrides import has_torch_function
 
 from . import _lib
 from ._util import require_dtype, require_gpu, stream_of
@@ -90,12 +94,21 @@ def _few_rows(rows: int, n: int, k: int) -> bool:
     return rows <= LINEAR_MAX_ROWS and k < 8192
 
 
+def _plain(*tensors: torch.Tensor | None) -> bool:
+    """Whether nothing of torch's stands between a call of F.linear and its kernel:
+    no function mode or tensor subclass, dispatch mode, function transform,
+    forward-mode level or autocast (a call of the library passes all of them by)."""
+    return not (has_torch_function(tensors) or _len_torch_dispatch_stack() or peek_interpreter_stack() is not None
+                or forward_ad._current_level >= 0 or torch.is_autocast_enabled())
+
+
 def _takes(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:
     """Whether ``linear`` runs on the few-row kernel."""
     rows, k = x.shape
     n = weight.shape[0]
     return not (weight.dim() != 2 or rows == 0 or n == 0 or not 0 < k <= LINEAR_MAX_K
                 or not _few_rows(rows, n, k) or n % 16 or k % 64 or not x.is_cuda
+                or not _plain(x, weight, bias)
                 or x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.device != x.device
                 or weight.shape[1] != k or not weight.is_contiguous() or x.stride(1) != 1 or x.stride(0) % 8
                 or x.stride(0) < k or rows * x.stride(0) > LINEAR_MAX_SPAN or x.data_ptr() % 16 or weight.data_ptr() % 16

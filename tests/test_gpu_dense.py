@@ -241,17 +241,69 @@ def test_few_row_linear_silu_routes(dev):
 def test_few_row_linear_leaves_what_the_kernel_refuses_to_torch(dev):
     """Rows whose stride spans more than mi_linear's 2^29 elements, and weights of
     no rows, no columns or one axis, are F.linear's."""
-    from minimal_inference_amd.dense import linear, linear_silu, silu_mul
+    from minimal_inference_amd.dense import _takes, linear
 
+    # (not multiplied: how the library takes rows this far apart is its own matter)
     step, k = (1 << 28) + 8, 512
     far = torch.zeros(step + k, device=dev, dtype=torch.bfloat16)
     x = far.as_strided((2, k), (step, 1))
-    x.copy_(torch.randn(2, k, device=dev))
     w = torch.randn(256, k, device=dev).to(torch.bfloat16)
-    assert torch.equal(linear(x, w), F.linear(x, w))
-    assert torch.equal(linear_silu(x, w), silu_mul(F.linear(x, w)))
+    assert not _takes(x, w, None) and _takes(far.as_strided((2, k), (step - 8, 1)), w, None)
+    x.copy_(torch.randn(2, k, device=dev))
     near = x.contiguous()
     assert torch.equal(linear(near, w[:0]), F.linear(near, w[:0]))
     assert torch.equal(linear(near, w[0]), F.linear(near, w[0]))
     for ww in (w[:, :0], torch.empty(256, 0, device=dev, dtype=torch.bfloat16)):
         assert torch.equal(linear(near[:, :0], ww), torch.zeros(2, 256, device=dev, dtype=torch.bfloat16))
+
+
+def test_few_row_linear_under_torchs_modes(dev):
+    """What torch does around F.linear happens around dense.linear too: autocast,
+    forward-mode tangents, function transforms, dispatch and function modes and
+    tensor subclasses all get F.linear's call."""
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from minimal_inference_amd.dense import _takes, linear
+
+    x = torch.randn(8, 512, device=dev).to(torch.bfloat16)
+    w = torch.randn(256, 512, device=dev).to(torch.bfloat16)
+    assert _takes(x, w, None)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert torch.equal(linear(x, w), F.linear(x, w)) and linear(x, w).dtype == torch.float16
+    with forward_ad.dual_level():
+        primal, tangent = forward_ad.unpack_dual(linear(x, forward_ad.make_dual(w, torch.ones_like(w))))
+        assert torch.equal(primal, F.linear(x, w)) and torch.equal(tangent, F.linear(x, torch.ones_like(w)))
+
+    def rows(xx):  # (the product itself would be a batched one)
+        assert not _takes(xx, w, None)
+        return xx
+
+    torch.vmap(rows)(x.view(2, 4, 512))
+
+    class Seen(TorchDispatchMode):
+        ops = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops += 1
+            return func(*args, **(kwargs or {}))
+
+    class Called(TorchFunctionMode):
+        linears = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.linears += func is F.linear
+            return func(*args, **(kwargs or {}))
+
+    class Named(torch.Tensor):
+        pass
+
+    with Seen() as seen:
+        linear(x, w)
+    with Called() as called:
+        linear(x, w)
+    assert seen.ops >= 1 and called.linears == 1
+    assert isinstance(linear(x, w.as_subclass(Named)), Named)
+    assert not _takes(x.as_subclass(Named), w, None) and not _takes(x, w, w[:, 0].contiguous().as_subclass(Named))
+    assert _takes(x, torch.nn.Parameter(w, requires_grad=False), None)
