@@ -115,16 +115,19 @@ struct SiluMulParams {
   int64_t rows;
 };
 
-// One thread per 8 outputs (16 bytes of g, of u and of out) of a row; the grid's
-// second axis walks the rows.  Bound: HBM.  With the scaled division, the software
-// roundings and an index division per thread it was VALU bound: 18,240 x 14,336
-// 318 us = 4.9 TB/s, now 272 us = 5.8 TB/s; 8,000 x 29,568 277 -> 234 us; 2,000 x
-// 14,336 35 -> 30 us.  (1,024 or 4,096 workgroup rows that walk further cost 17 %
-// and 9 %; the reciprocal without its two steps gains 4 %.)
-__global__ __launch_bounds__(256) void silu_mul_kernel(SiluMulParams p) {
-  const int ch = int(blockIdx.x) * 256 + threadIdx.x;
+// One thread per 8 outputs (16 bytes of g, of u and of out) of a row; a workgroup
+// is blockDim.y rows of blockDim.x chunks, and the grid's second axis walks the
+// rows.  Bound: HBM.  With the scaled division, the software roundings and an index
+// division per thread it was VALU bound: 18,240 x 14,336 295-318 us = 4.9 TB/s, now
+// 251-272 us = 5.8 TB/s; 8,000 x 29,568 277 -> 234 us; 2,000 x 14,336 35 -> 30 us.
+// (1,024 or 4,096 workgroup rows that walk further cost 17 % and 9 %; the reciprocal
+// without its two steps gains 4 %.)
+constexpr int kSiluThreads = 256;
+__global__ __launch_bounds__(kSiluThreads) void silu_mul_kernel(SiluMulParams p) {
+  const int ch = int(blockIdx.x * blockDim.x + threadIdx.x);
   if (ch * 8 >= p.inter) return;
-  for (int64_t row = blockIdx.y; row < p.rows; row += gridDim.y) {
+  const int64_t step = int64_t(gridDim.y) * blockDim.y;
+  for (int64_t row = int64_t(blockIdx.y) * blockDim.y + threadIdx.y; row < p.rows; row += step) {
     const uint16_t* g = p.gu + row * p.gu_stride + ch * 8;
     const uint4 gv = mi::load16_nt(g), uv = mi::load16_nt(g + p.inter);
     const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
@@ -190,8 +193,15 @@ extern "C" int mi_silu_mul(const void* gate_up, int64_t gate_up_stride, void* ou
   p.o_stride = out_stride;
   p.inter = intermediate;
   p.rows = rows;
-  if (rows > 0x7fffffff * int64_t(256) / (intermediate / 8)) return mi::fail(MI_ERR_INVALID, "silu_mul: too many rows");
-  const dim3 grid(uint32_t((intermediate / 8 + 255) / 256), uint32_t(std::min<int64_t>(rows, 65535)));
-  hipLaunchKernelGGL(silu_mul_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
+  if (rows > 0x7fffffff * int64_t(256) / (intermediate / 8))  // (refused since the grid had one axis)
+    return mi::fail(MI_ERR_INVALID, "silu_mul: too many rows");
+  // Rows of up to two workgroups' chunks are dealt evenly, as many of them to a
+  // workgroup as it has threads for (one workgroup row per row: 100,000 x 64 44 us,
+  // now 9.4; 18,240 x 768 20.2, 16.6; 18,240 x 2,816 62, 50); longer ones take whole
+  // workgroups and the rest (18,240 x 4,864 85 us, dealt evenly 99; with 512 threads 89).
+  const int chunks = intermediate / 8, parts = (chunks + kSiluThreads - 1) / kSiluThreads;
+  const int bx = parts > 2 ? kSiluThreads : (chunks + parts - 1) / parts, by = kSiluThreads / bx;
+  const dim3 grid(parts, uint32_t(std::min<int64_t>((rows + by - 1) / by, 65535)));
+  hipLaunchKernelGGL(silu_mul_kernel, grid, dim3(bx, by), 0, static_cast<hipStream_t>(stream), p);
   return mi::check_launch("silu_mul_kernel");
 }

@@ -307,3 +307,22 @@ def test_few_row_linear_under_torchs_modes(dev):
     assert isinstance(linear(x, w.as_subclass(Named)), Named)
     assert not _takes(x.as_subclass(Named), w, None) and not _takes(x, w, w[:, 0].contiguous().as_subclass(Named))
     assert _takes(x, torch.nn.Parameter(w, requires_grad=False), None)
+
+
+@pytest.mark.parametrize("rows,inter", [
+    *[(rows, inter) for inter in (8, 16, 40, 1000, 2040, 2048, 2056, 2816, 4096, 4104, 4864) for rows in (1, 3, 31, 257)],
+    (65535 + 70, 1032), (2 * 65535 + 3, 1024)])
+def test_silu_mul_widths(dev, rows, inter):
+    """The shapes of a workgroup (many rows, one, half of one, part of one), rows that
+    do not fill the last, and more workgroups of rows than the grid's second axis
+    has: the bits of the fp32 formula, nothing written around them."""
+    from minimal_inference_amd.dense import silu_mul
+
+    g = torch.Generator(device=dev).manual_seed(rows * 131 + inter)
+    gu = (3 * torch.randn(rows, 2 * inter, device=dev, generator=g)).to(torch.bfloat16)
+    out = torch.full((rows + 1, inter + 8), 7.0, device=dev, dtype=torch.bfloat16)
+    silu_mul(gu, out=out[:rows, :inter])
+    gate, up = gu[:, :inter].float(), gu[:, inter:].float()
+    ref = ((gate / (1 + torch.exp(-gate))).to(torch.bfloat16).float() * up).to(torch.bfloat16)
+    assert torch.equal(out[:rows, :inter], ref)
+    assert bool((out[rows] == 7.0).all()) and bool((out[:, inter:] == 7.0).all())
