@@ -48,11 +48,16 @@ __host__ __device__ constexpr int split_groups(int nsplit, int direct) {
   const int n = (nsplit + per - 1) / per;
   return n < kMaxGroups ? n : kMaxGroups;
 }
-// Three round trips while a 16-byte load per lane covers the rows of all of a
-// KV head's Q heads (19 splits, Mistral-7B heads B=4: direct 10.7 us, two
-// levels 11.0), two when it takes more loads (Qwen2.5-7B heads B=8, up to 24
-// splits: 13.8 and 13.1).
-__host__ __device__ constexpr int direct_splits(int head_dim, int group) { return group * head_dim > 512 ? 16 : 24; }
+// head_dim 128 and 256: three round trips while a 16-byte load per lane covers the
+// rows of all of a KV head's Q heads (19 splits, Mistral-7B heads B=4: direct 10.7
+// us, two levels 11.0), two when it takes more loads (Qwen2.5-7B heads B=8, up to
+// 24 splits: 13.8 and 13.1).  head_dim 64, whose merge keeps a further round trip
+// on its way: 25 splits, Qwen2.5-0.5B heads B=1, direct 7.8 us, two levels 8.4 (one
+// KV head of 8: 7.0, 7.8); 32 splits 8.2, 8.4 (7.3, 7.9); 40 splits 9.1, 8.6 (8.0,
+// 7.9).
+__host__ __device__ constexpr int direct_splits(int head_dim, int group) {
+  return head_dim == 64 ? 36 : group * head_dim > 512 ? 16 : 24;
+}
 constexpr int kPlanThreads = 1024;  // both planning kernels run one workgroup of this size
 
 // One item = a contiguous page range of one request.  Read by a wave with one

@@ -371,13 +371,14 @@ def test_repeated_runs_are_bit_identical(dev, parity, hq, hkv, d, lo, hi):
 
 
 # (heads, context): one request; head_dim 128 merges up to 24 splits in one
-# level with groups of up to 4 Q heads and 16 with more, head_dim 64 24, 256 by
+# level with groups of up to 4 Q heads and 16 with more, head_dim 64 36, 256 by
 # how many 16-byte loads its heads take
 @pytest.mark.parametrize("hq,hkv,d,ctx,nsplit", [
     (32, 8, 128, 16 * 64 - 3, 16), (32, 8, 128, 16 * 96, 24), (32, 8, 128, 16 * 97 + 5, 25),  # the last direct one
     (28, 4, 128, 16 * 64, 16), (28, 4, 128, 16 * 65, 17), (64, 8, 128, 16 * 256 - 15, 59),  # (the other requests take their part of the units)
     (8, 1, 128, 16 * 257, 65), (5, 1, 128, 16 * 1024 - 1, 256), (6, 1, 128, 16 * 1028 + 1, 258),  # groups of 16, of 24
     (14, 2, 64, 16 * 100, 25), (4, 1, 64, 32768, 505), (2, 2, 64, 16 * 260, 65),
+    (14, 2, 64, 16 * 144, 36), (14, 2, 64, 16 * 148, 37), (8, 1, 64, 16 * 144 - 9, 36), (8, 1, 64, 16 * 147 + 1, 37),
     (16, 4, 256, 16 * 65, 17), (4, 2, 256, 16 * 100, 25), (8, 1, 256, 16 * 900, 225),
 ])
 def test_splits_merged_in_two_levels(dev, parity, hq, hkv, d, ctx, nsplit):
