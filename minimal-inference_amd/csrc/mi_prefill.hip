@@ -139,9 +139,9 @@ size_t prefill_ws_bytes(int batch, int64_t total_q) {
   return 256 + mi::align_up(tile_capacity(batch, total_q) * sizeof(PrefillTile), 256);
 }
 
-// Workgroups resident at once: two per CU at head_dim 128 (registers), three
-// at 64, one at 256 (LDS).
-int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 3 : head_dim == 128 ? 2 : 1); }
+// Workgroups resident at once: two per CU at head_dim 128 and four at 64
+// (registers: run_waves), one at 256 (LDS).
+int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 4 : head_dim == 128 ? 2 : 1); }
 
 // Fine tiles are for launches that leave most of the chip idle: a KV tile
 // takes a workgroup of one row block per wave 1.1-1.3 us instead of the 2.2-2.8
@@ -151,9 +151,10 @@ int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 3 :
 // (and split): one prompt of 512 tokens 23.9 / 21.8 / 13.5 us, 1,024: 41.0 /
 // 36.2 / 25.3, 64 new tokens on 8,000 cached 267 / 66.5 / 31.7; 2,048: 79 / 54 /
 // 60; four turns of 61-413 tokens on 2,000-6,000 cached 199 / 89 / 132;
-// Qwen2.5-7B heads, one prompt of 1,537: 59 / 41 / 44.  So: fine while the load per resident workgroup, counted in fine KV
-// tiles, is at most kFineLoad.
-constexpr int kFineLoad = 12;
+// Qwen2.5-7B heads, one prompt of 1,537: 59 / 41 / 44.  So: fine while the load per
+// resident workgroup, counted in fine KV tiles, is at most fine_load: 12, or at
+// head_dim 64, with twice the workgroups, 9.
+constexpr float fine_load(int head_dim) { return head_dim == 64 ? 9.f : 12.f; }
 constexpr int kFineRounds = 4;  // resident rounds of fine units at most
 
 // Workgroups of the run: whole resident rounds over the most coarse tiles the
@@ -230,6 +231,7 @@ struct PlanParams {
   int bm[2], blocks[2], slots[2];  // positions, row blocks per wave and partial slots of fine [0] and coarse [1] tiles
   size_t counters_off[2];          // of the merge counters, behind the partials
   int resident;                    // workgroups resident at once
+  float fine_load;
   int tile_room;                   // tiles the list holds in front of the units
   int unit_capacity;               // 0: tiles only
   char* ws;
@@ -430,10 +432,10 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
     return (max(0, min(x.kv_len, x.row0 + x.q_rows + x.kv_len - x.qo_len)) + kKvTile - 1) / kKvTile;
   };
   for (int i = t; i < fit; i += kPlanThreads) p.tiles[i] = tile_of(i);
-  // fine or coarse units (see kFineLoad)
+  // fine or coarse units (see fine_load)
   const bool room = p.unit_capacity > 0 && ntiles == fit && fit <= p.tile_room;
-  const float fine_load = area * float(p.group * p.hkv) / (64.f * kKvTile * float(p.resident));
-  const int form = room && p.blocks[1] > 1 && fine_load <= float(kFineLoad) &&
+  const float load = area * float(p.group * p.hkv) / (64.f * kKvTile * float(p.resident));
+  const int form = room && p.blocks[1] > 1 && load <= p.fine_load &&
                            fine_tiles * float(p.hkv) <= float(kFineRounds * p.resident) ? 0 : 1;
   const int nslots = p.slots[form];
   if (form == 0) {
@@ -675,7 +677,8 @@ struct PartialArea {
 // different XCDs; the counter is back at zero for the next run of the plan.
 // What bounds a merge is the round trip of its reads (104 KB per split at
 // head_dim 128): the wave walks (row block, split) as one sequence with DP
-// row blocks on their way.
+// row blocks on their way (four of them at head_dim 64 would take the whole
+// kernel from four waves per SIMD to three).
 template <int D, int MAXRB>
 __device__ __forceinline__ bool merge_splits(const RunParams& p, int part, const PartialArea& pa, int hkv, int w, int lane, int nblk,
                                              lds_t* lds, lds_t* ob, const mi::f32x4_t (&o)[MAXRB][D / 16],
@@ -683,7 +686,7 @@ __device__ __forceinline__ bool merge_splits(const RunParams& p, int part, const
   using T = PrefillTraits<D, MAXRB>;
   constexpr int NT = T::NT;
   constexpr int CP = 16;  // cache policy: sc1 (device scope)
-  constexpr int DP = D == 256 ? 1 : MAXRB == 3 ? 3 : 4;
+  constexpr int DP = D == 256 ? 1 : MAXRB == 3 || D == 64 ? 3 : 4;
   constexpr int WB = MAXRB * (NT * 1024 + 512);  // bytes of one wave's partial
   static_assert(WB * T::WAVES == int(partial_bytes(D, MAXRB)), "partial layout");
   const int g = lane >> 4;
@@ -1185,10 +1188,14 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
   }
 }
 
+// Waves per SIMD of the run.  head_dim 64 keeps four (125 registers): with three,
+// 832 tiles of short prompts took 9.3 us instead of 7.3.
+constexpr int run_waves(int head_dim) { return head_dim == 64 ? 4 : head_dim == 128 ? 2 : 1; }
+
 // The units of the plan if this run may take them, else its tiles.  The plan
 // says which form the units have: coarse, RB row blocks per wave, or fine, one.
 template <int D, int RB>
-__global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 2 : 1))) void prefill_run_kernel(RunParams p) {
+__global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_eu(run_waves(D)))) void prefill_run_kernel(RunParams p) {
   __shared__ __attribute__((aligned(16))) char smem[PrefillTraits<D, RB>::SMEM];  // [buffer][K, V], then the output rows
   static_assert(PrefillTraits<D, 1>::SMEM <= PrefillTraits<D, RB>::SMEM, "LDS of the fine form");
   lds_t* lds = (lds_t*)smem;
@@ -1253,6 +1260,7 @@ extern "C" int mi_prefill_plan(void* workspace, size_t workspace_bytes, const in
   pp.group = num_qo_heads / num_kv_heads;
   pp.hkv = num_kv_heads;
   pp.resident = resident_groups(head_dim);
+  pp.fine_load = fine_load(head_dim);
   const UnitLayout L = unit_layout(workspace_bytes, num_kv_heads, head_dim);
   static std::atomic<uint64_t> plans{0};
   pp.serial = (plans.fetch_add(1, std::memory_order_relaxed) + 1) * 0x9e3779b97f4a7c15ull;
