@@ -154,6 +154,18 @@ int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 4 :
 // Qwen2.5-7B heads, one prompt of 1,537: 59 / 41 / 44.  So: fine while the load per
 // resident workgroup, counted in fine KV tiles, is at most fine_load: 12, or at
 // head_dim 64, with twice the workgroups, 9.
+//
+// Fine tiles of more than one resident round must pay for the rounds as well: they
+// are taken only where rows and longest chain make them no slower than coarse
+// tiles at the same cost per KV tile, load + longest / 2 <= max(longest, load +
+// longest / 2) with the loads in each form's own tiles (a chain is on average
+// half the longest when it starts).  Of 500 launches of 1-64 requests with up to
+// four rounds of fine tiles, 18 of head_dim 128 were up to 20 % slower in fine
+// tiles than in the whole coarse ones (32 requests of 20 rows on 500 cached,
+// Qwen2.5-72B heads, 27.3 / 32.2 us; 32 of 300 on 100, 8 KV heads of one, 31.6 /
+// 34.3), with this line three, by at most 7 %.  Coarse tiles of a launch below the load line are
+// not split: at few KV tiles per workgroup the partials of three row blocks cost
+// more than the chain (five prompts of 307, Qwen2.5-7B heads, 17.5 whole, 25.3 split).
 constexpr float fine_load(int head_dim) { return head_dim == 64 ? 9.f : 12.f; }
 constexpr int kFineRounds = 4;  // resident rounds of fine units at most
 
@@ -231,6 +243,7 @@ struct PlanParams {
   int bm[2], blocks[2], slots[2];  // positions, row blocks per wave and partial slots of fine [0] and coarse [1] tiles
   size_t counters_off[2];          // of the merge counters, behind the partials
   int resident;                    // workgroups resident at once
+  int head_dim;
   float fine_load;
   int tile_room;                   // tiles the list holds in front of the units
   int unit_capacity;               // 0: tiles only
@@ -246,6 +259,15 @@ struct PlanParams {
 constexpr int kPlanThreads = 1024;
 constexpr int kSplitTiles = 8192;  // most query tiles whose keys are considered for splitting
 constexpr int kMinChunk = 4;  // KV tiles per unit at least (2 and 3 measured the same on a 512-token prompt)
+// KV tiles that splitting must take off the longest chain: the partials cost about
+// as much as two, and where the units take half of the resident workgroups' places
+// or more, they share the CUs and the merges with the others.  (us, whole / split:
+// 16 requests of 16 rows on 300 cached, head_dim 256, five KV tiles to four, 16.2 /
+// 18.2; Mistral-7B heads 9.9 / 11.6; 20 of 10 on 400, seven to four, 12.9 / 15.5; 32
+// of 20 on 500, 16 KV heads of one, head_dim 64, nine to five, 15.5 / 20.8.  One row on
+// 400 cached, seven to four, most of the chip idle, 11.9 / 11.0; head_dim 256, one
+// workgroup per CU in any case, 512 tokens 22.3 / 18.9.)
+constexpr int kMinSaved = 2, kMinSavedCrowded = 5;
 
 // Inclusive scan over the block: shuffles inside each wave, then the wave
 // totals through LDS.  *total gets the block-wide sum.
@@ -354,6 +376,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
   __shared__ int s_qo[kPlanThreads], s_kv[kPlanThreads], s_q0[kPlanThreads], s_pb0[kPlanThreads];
   __shared__ int s_req[kPlanThreads], s_end[kPlanThreads], wsum[kPlanThreads / 64];
   __shared__ int red[2][kPlanThreads / 64], ok[2][kPlanThreads / 64], s_fit;
+  __shared__ float s_sums[4][kPlanThreads / 64];
   __shared__ unsigned short s_n[kSplitTiles];
   if (p.batch > kPlanThreads) {
     plan_large(p, wsum);
@@ -362,7 +385,11 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   constexpr int NW = kPlanThreads / 64;
   int qo = 0;
-  float area = 0.f, fine_tiles = 0.f;  // this request's (row, key) pairs with half a KV tile of masked ones per row
+  // this request's (row, key) pairs with half a KV tile of masked ones per row, its
+  // fine tiles, and the KV tiles of its fine and its coarse ones
+  enum { kArea, kFineTiles, kFineKv, kCoarseKv, kSums };
+  float sums[kSums] = {};
+  int most_kv = 0;
   if (t < p.batch) {
     const int q0 = p.qo_indptr[t], q1 = p.qo_indptr[t + 1], pb0 = p.kv_indptr[t], pb1 = p.kv_indptr[t + 1];
     const int lpl = p.last_page_len[t];
@@ -373,24 +400,36 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
     s_q0[t] = q0;
     s_pb0[t] = pb0;
     s_kv[t] = kv;
-    area = float(qo) * (max(0.f, float(kv) - 0.5f * float(qo)) + 0.5f * kKvTile);
-    fine_tiles = float((qo + p.bm[0] - 1) / p.bm[0]);
+    const float keys = max(0.f, float(kv) - 0.5f * float(qo)) + 0.5f * kKvTile;  // of a row, on average
+    sums[kArea] = float(qo) * keys;
+    sums[kFineTiles] = float((qo + p.bm[0] - 1) / p.bm[0]);
+    sums[kFineKv] = sums[kFineTiles] * keys * (1.f / kKvTile);
+    sums[kCoarseKv] = float((qo + p.bm[1] - 1) / p.bm[1]) * keys * (1.f / kKvTile);
+    most_kv = qo > 0 ? kv : 0;
   }
+  const int request_waves = (p.batch + 63) / 64;  // (the others would only slow these down)
+  if (w < request_waves) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    area += __shfl_xor(area, o);
-    fine_tiles += __shfl_xor(fine_tiles, o);
-  }
-  if (lane == 0) {
-    red[0][w] = __float_as_int(area);
-    red[1][w] = __float_as_int(fine_tiles);
+    for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+      for (int k = 0; k < kSums; ++k) sums[k] += __shfl_xor(sums[k], o);
+      most_kv = max(most_kv, __shfl_xor(most_kv, o));
+    }
+    if (lane == 0) {
+#pragma unroll
+      for (int k = 0; k < kSums; ++k) s_sums[k][w] = sums[k];
+      red[0][w] = most_kv;
+    }
   }
   if (t == 0) s_fit = 0;
   __syncthreads();
-  area = fine_tiles = 0.f;
-  for (int i = 0; i < NW; ++i) {
-    area += __int_as_float(red[0][i]);
-    fine_tiles += __int_as_float(red[1][i]);
+#pragma unroll
+  for (int k = 0; k < kSums; ++k) sums[k] = 0.f;
+#pragma nounroll
+  for (int i = 0; i < request_waves; ++i) {
+#pragma unroll
+    for (int k = 0; k < kSums; ++k) sums[k] += s_sums[k][i];
+    most_kv = max(most_kv, red[0][i]);
   }
   int rank = 0;
   for (int c = 0; c < p.batch; ++c) {
@@ -434,9 +473,12 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
   for (int i = t; i < fit; i += kPlanThreads) p.tiles[i] = tile_of(i);
   // fine or coarse units (see fine_load)
   const bool room = p.unit_capacity > 0 && ntiles == fit && fit <= p.tile_room;
-  const float load = area * float(p.group * p.hkv) / (64.f * kKvTile * float(p.resident));
-  const int form = room && p.blocks[1] > 1 && load <= p.fine_load &&
-                           fine_tiles * float(p.hkv) <= float(kFineRounds * p.resident) ? 0 : 1;
+  const float per_group = float(p.hkv) / float(p.resident), chain = float((most_kv + kKvTile - 1) / kKvTile);
+  const bool light = sums[kArea] * float(p.group) * per_group <= 64.f * kKvTile * p.fine_load;
+  const float rounds_fine = sums[kFineTiles] * per_group;
+  const bool even = sums[kFineKv] * per_group + 0.5f * chain <= max(chain, sums[kCoarseKv] * per_group + 0.5f * chain);
+  const int form =
+      room && p.blocks[1] > 1 && light && rounds_fine <= float(kFineRounds) && (rounds_fine <= 1.f || even) ? 0 : 1;
   const int nslots = p.slots[form];
   if (form == 0) {
     __syncthreads();  // s_end's readers are done
@@ -446,7 +488,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
   // the units that fill the rounds which the unsplit tiles need
   const int rounds = (ntiles * p.hkv + p.resident - 1) / p.resident;
   const int limit = min(rounds * p.resident / p.hkv, p.unit_capacity);
-  const bool consider = room && (form == 0 || rounds == 1) && ntiles <= min(kSplitTiles, limit);
+  const bool consider = room && (form == 0 || (rounds == 1 && (!light || p.blocks[1] == 1))) && ntiles <= min(kSplitTiles, limit);
   int chunk = 0, longest = 0;
   if (consider) {
     int sum = 0;
@@ -500,7 +542,9 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
         lo = nlo;
         hi = nhi;
       }
-      chunk = lo < longest ? lo : 0;
+      // (kMinSaved)
+      const bool crowded = (float(total) / float(lo) + 0.5f * float(ntiles)) * per_group >= 0.5f;
+      chunk = lo + (crowded && p.head_dim <= 128 ? kMinSavedCrowded : kMinSaved) <= longest ? lo : 0;
     }
   }
   // whole fine tiles are units, whole coarse ones the tiles that are listed already
@@ -1260,6 +1304,7 @@ extern "C" int mi_prefill_plan(void* workspace, size_t workspace_bytes, const in
   pp.group = num_qo_heads / num_kv_heads;
   pp.hkv = num_kv_heads;
   pp.resident = resident_groups(head_dim);
+  pp.head_dim = head_dim;
   pp.fine_load = fine_load(head_dim);
   const UnitLayout L = unit_layout(workspace_bytes, num_kv_heads, head_dim);
   static std::atomic<uint64_t> plans{0};
