@@ -139,9 +139,11 @@ size_t prefill_ws_bytes(int batch, int64_t total_q) {
   return 256 + mi::align_up(tile_capacity(batch, total_q) * sizeof(PrefillTile), 256);
 }
 
-// Workgroups resident at once: two per CU at head_dim 128 and four at 64
-// (registers: run_waves), one at 256 (LDS).
-int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 4 : head_dim == 128 ? 2 : 1); }
+// Workgroups resident at once, as the plan counts them: two per CU at head_dim 128
+// (registers), one at 256 (LDS), three of the four that fit at 64 (filling the
+// fourth place with splits, one prompt of 1,537 tokens, Qwen2.5-0.5B heads, took
+// 19.6 us instead of 15.7).
+int resident_groups(int cus, int head_dim) { return cus * (head_dim == 64 ? 3 : head_dim == 128 ? 2 : 1); }
 
 // Fine tiles are for launches that leave most of the chip idle: a KV tile
 // takes a workgroup of one row block per wave 1.1-1.3 us instead of the 2.2-2.8
@@ -152,8 +154,7 @@ int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 4 :
 // 36.2 / 25.3, 64 new tokens on 8,000 cached 267 / 66.5 / 31.7; 2,048: 79 / 54 /
 // 60; four turns of 61-413 tokens on 2,000-6,000 cached 199 / 89 / 132;
 // Qwen2.5-7B heads, one prompt of 1,537: 59 / 41 / 44.  So: fine while the load per
-// resident workgroup, counted in fine KV tiles, is at most fine_load: 12, or at
-// head_dim 64, with twice the workgroups, 9.
+// resident workgroup, counted in fine KV tiles, is at most kFineLoad.
 //
 // Fine tiles of more than one resident round must pay for the rounds as well: they
 // are taken only where rows and longest chain make them no slower than coarse
@@ -166,14 +167,13 @@ int resident_groups(int head_dim) { return mi::num_cus() * (head_dim == 64 ? 4 :
 // 34.3), with this line three, by at most 7 %.  Coarse tiles of a launch below the load line are
 // not split: at few KV tiles per workgroup the partials of three row blocks cost
 // more than the chain (five prompts of 307, Qwen2.5-7B heads, 17.5 whole, 25.3 split).
-constexpr float fine_load(int head_dim) { return head_dim == 64 ? 9.f : 12.f; }
+constexpr int kFineLoad = 12;
 constexpr int kFineRounds = 4;  // resident rounds of fine units at most
 
 // Workgroups of the run: whole resident rounds over the most coarse tiles the
 // rows can make, or the units that a plan of fine tiles may hold.  The plan
 // never makes more.
-int64_t run_groups(int batch, int64_t total_q, int group, int hkv, int head_dim) {
-  const int64_t res = resident_groups(head_dim);
+int64_t run_groups(int64_t res, int batch, int64_t total_q, int group, int hkv, int head_dim) {
   const auto groups = [&](int blocks) { return (total_q / rows_per_tile(group, head_dim, blocks) + batch) * hkv; };
   const int64_t coarse = (groups(row_blocks(head_dim)) + res - 1) / res * res;
   const int64_t fine = (groups(1) + res - 1) / res * res;
@@ -199,13 +199,13 @@ struct UnitLayout {
   size_t off, parts;
   int capacity, coarse, fine;
 };
-UnitLayout unit_layout(size_t workspace_bytes, int hkv, int head_dim) {
+UnitLayout unit_layout(int res, size_t workspace_bytes, int hkv, int head_dim) {
   const auto per = [&](int blocks) { return (partial_bytes(head_dim, blocks) + kCounterStride * sizeof(int)) * size_t(hkv); };
   UnitLayout L{0, 0, 0, 0, 0};
   const size_t coarse = per(row_blocks(head_dim)), limit = workspace_bytes / 4 * 3;
-  const int capacity = kFineRounds * resident_groups(head_dim) / hkv;
+  const int capacity = kFineRounds * res / hkv;
   const size_t list = 256 + mi::align_up(size_t(capacity) * sizeof(PrefillTile), 256);
-  const size_t c = limit < list ? 0 : std::min((limit - list) / coarse, size_t(2 * resident_groups(head_dim) / hkv));
+  const size_t c = limit < list ? 0 : std::min((limit - list) / coarse, size_t(2 * res / hkv));
   if (c < 2 || list + c * coarse + 512 + sizeof(PrefillTile) > workspace_bytes) return L;
   L.off = (workspace_bytes - c * coarse - list) & ~size_t(255);
   L.parts = L.off + list;
@@ -243,8 +243,7 @@ struct PlanParams {
   int bm[2], blocks[2], slots[2];  // positions, row blocks per wave and partial slots of fine [0] and coarse [1] tiles
   size_t counters_off[2];          // of the merge counters, behind the partials
   int resident;                    // workgroups resident at once
-  int head_dim;
-  float fine_load;
+  int cus;                         // their number, where several workgroups share one (0: one each)
   int tile_room;                   // tiles the list holds in front of the units
   int unit_capacity;               // 0: tiles only
   char* ws;
@@ -260,14 +259,12 @@ constexpr int kPlanThreads = 1024;
 constexpr int kSplitTiles = 8192;  // most query tiles whose keys are considered for splitting
 constexpr int kMinChunk = 4;  // KV tiles per unit at least (2 and 3 measured the same on a 512-token prompt)
 // KV tiles that splitting must take off the longest chain: the partials cost about
-// as much as two, and where the units take half of the resident workgroups' places
-// or more, they share the CUs and the merges with the others.  (us, whole / split:
-// 16 requests of 16 rows on 300 cached, head_dim 256, five KV tiles to four, 16.2 /
-// 18.2; Mistral-7B heads 9.9 / 11.6; 20 of 10 on 400, seven to four, 12.9 / 15.5; 32
-// of 20 on 500, 16 KV heads of one, head_dim 64, nine to five, 15.5 / 20.8.  One row on
-// 400 cached, seven to four, most of the chip idle, 11.9 / 11.0; head_dim 256, one
-// workgroup per CU in any case, 512 tokens 22.3 / 18.9.)
-constexpr int kMinSaved = 2, kMinSavedCrowded = 5;
+// as much as two, and more where the whole tiles had a CU each and the units share
+// them.  (us, whole / split: 16 requests of 16 rows on 300 cached, head_dim 256, five
+// KV tiles to four, 16.2 / 18.2; Mistral-7B heads 9.9 / 11.6; 20 of 10 on 400, seven
+// to four, 12.9 / 15.5.  One row on 400 cached, seven to four, most of the chip idle,
+// 11.9 / 11.0; 900 tokens, Qwen2.5-7B heads, 15 to 12, 400 tiles, 23.5 / 19.0.)
+constexpr int kMinSaved = 2, kMinSavedCrowd = 5;
 
 // Inclusive scan over the block: shuffles inside each wave, then the wave
 // totals through LDS.  *total gets the block-wide sum.
@@ -471,10 +468,10 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
     return (max(0, min(x.kv_len, x.row0 + x.q_rows + x.kv_len - x.qo_len)) + kKvTile - 1) / kKvTile;
   };
   for (int i = t; i < fit; i += kPlanThreads) p.tiles[i] = tile_of(i);
-  // fine or coarse units (see fine_load)
+  // fine or coarse units (see kFineLoad)
   const bool room = p.unit_capacity > 0 && ntiles == fit && fit <= p.tile_room;
   const float per_group = float(p.hkv) / float(p.resident), chain = float((most_kv + kKvTile - 1) / kKvTile);
-  const bool light = sums[kArea] * float(p.group) * per_group <= 64.f * kKvTile * p.fine_load;
+  const bool light = sums[kArea] * float(p.group) * per_group <= 64.f * kKvTile * float(kFineLoad);
   const float rounds_fine = sums[kFineTiles] * per_group;
   const bool even = sums[kFineKv] * per_group + 0.5f * chain <= max(chain, sums[kCoarseKv] * per_group + 0.5f * chain);
   const int form =
@@ -543,8 +540,9 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
         hi = nhi;
       }
       // (kMinSaved)
-      const bool crowded = (float(total) / float(lo) + 0.5f * float(ntiles)) * per_group >= 0.5f;
-      chunk = lo + (crowded && p.head_dim <= 128 ? kMinSavedCrowded : kMinSaved) <= longest ? lo : 0;
+      const bool crowd = float(ntiles * p.hkv) <= float(p.cus) &&
+                         (float(total) / float(lo) + 0.5f * float(ntiles)) * float(p.hkv) > float(p.cus);
+      chunk = lo + (crowd ? kMinSavedCrowd : kMinSaved) <= longest ? lo : 0;
     }
   }
   // whole fine tiles are units, whole coarse ones the tiles that are listed already
@@ -590,6 +588,8 @@ struct RunParams {
   const uint64_t* unit_serial;
   char* parts;
   RunKey key;
+  int last_tile, last_unit;       // of the room of either list
+  int max_units;                  // that the grid covers
   int tile_bm;                    // positions per coarse tile
   const uint16_t* q;
   int64_t q_st, q_sh;
@@ -1243,6 +1243,13 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
   __shared__ __attribute__((aligned(16))) char smem[PrefillTraits<D, RB>::SMEM];  // [buffer][K, V], then the output rows
   static_assert(PrefillTraits<D, 1>::SMEM <= PrefillTraits<D, RB>::SMEM, "LDS of the fine form");
   lds_t* lds = (lds_t*)smem;
+  // every argument from the argument segment at once: left to the compiler, some of
+  // these reads came after the header's, one more round trip each
+  __asm__ volatile("" ::"s"(p.header), "s"(p.tiles), "s"(p.units), "s"(p.unit_serial), "s"(p.parts), "s"(p.key.ws),
+                   "s"(p.key.bytes), "s"(p.key.stream), "s"(p.key.shape), "s"(p.last_tile), "s"(p.last_unit),
+                   "s"(p.max_units), "s"(p.tile_bm), "s"(p.q), "s"(p.q_st), "s"(p.q_sh), "s"(p.q_ext), "s"(p.pool),
+                   "s"(p.num_pages), "s"(p.indices), "s"(p.total_q), "s"(p.hkv), "s"(p.group), "s"(p.causal),
+                   "s"(p.scale_log2));
   const int tile_idx = int(blockIdx.x) / p.hkv;
   const int hkv = int(blockIdx.x) - tile_idx * p.hkv;
   // The header and the record (not written during the launch) are read through
@@ -1254,17 +1261,24 @@ __global__ __launch_bounds__(64 * waves_for(D)) __attribute__((amdgpu_waves_per_
   typedef __attribute__((address_space(4))) const int const_int;
   const const_header* h = (const const_header*)(p.header);
   typedef __attribute__((address_space(4))) const uint64_t const_u64;
-  // (without branches: the compiler then loads all of it in one round trip; one
-  // test after the other cost a run 0.7 us)
+  // Both lists' records (clamped into them) go out with the header, and the tests
+  // have no branches, so that all of it takes one round trip.
+  const const_int* fu = (const const_int*)(p.units + min(tile_idx, p.last_unit));
+  const const_int* ft = (const const_int*)(p.tiles + min(tile_idx, p.last_tile));
+  const PrefillTile tu{fu[0], fu[1], fu[2], fu[3], fu[4], fu[5], fu[6], fu[7]};
+  const PrefillTile tt{ft[0], ft[1], ft[2], ft[3], ft[4], ft[5], ft[6], ft[7]};
   const uint64_t serial = *(const const_u64*)(p.unit_serial);
   const int num_units = h->units, num_tiles = h->num_tiles, unit_bm = h->bm, blocks = h->row_blocks;
   const uint64_t differs = (h->key.ws ^ p.key.ws) | (h->key.bytes ^ p.key.bytes) | (h->key.stream ^ p.key.stream) |
                            (h->key.shape ^ p.key.shape) | (h->serial ^ serial) | uint64_t(p.key.stream == 0);
   const PartialArea pa{p.parts, h->slots};
-  const bool own = (num_units > 0) & (differs == 0) & (int64_t(num_units) * p.hkv <= int64_t(gridDim.x));
+  const bool own = (num_units > 0) & (differs == 0) & (num_units <= p.max_units);
+  const PrefillTile t{own ? tu.q_begin : tt.q_begin, own ? tu.q_rows : tt.q_rows, own ? tu.qo_len : tt.qo_len,
+                      own ? tu.kv_len : tt.kv_len,   own ? tu.row0 : tt.row0,     own ? tu.kv_page_begin : tt.kv_page_begin,
+                      own ? tu.kt : tt.kt,           own ? tu.part : tt.part};
+  __asm__ volatile("" ::"s"(t.q_begin), "s"(t.q_rows), "s"(t.qo_len), "s"(t.kv_len), "s"(t.row0), "s"(t.kv_page_begin),
+                   "s"(t.kt), "s"(t.part), "s"(unit_bm), "s"(blocks), "s"(pa.slots));  // (else their loads sink below the return)
   if (tile_idx >= (own ? num_units : num_tiles)) return;  // whole workgroup
-  const const_int* f = (const const_int*)((own ? p.units : p.tiles) + tile_idx);
-  const PrefillTile t{f[0], f[1], f[2], f[3], f[4], f[5], f[6], f[7]};
   const int bm = own ? unit_bm : p.tile_bm;
   if (RB > 1 && own && blocks == 1) run_unit<D, 1>(p, t, pa, hkv, bm, lds);
   else run_unit<D, RB>(p, t, pa, hkv, bm, lds);
@@ -1303,10 +1317,10 @@ extern "C" int mi_prefill_plan(void* workspace, size_t workspace_bytes, const in
   pp.capacity = int(tile_capacity(batch_size, total_q));
   pp.group = num_qo_heads / num_kv_heads;
   pp.hkv = num_kv_heads;
-  pp.resident = resident_groups(head_dim);
-  pp.head_dim = head_dim;
-  pp.fine_load = fine_load(head_dim);
-  const UnitLayout L = unit_layout(workspace_bytes, num_kv_heads, head_dim);
+  const int cus = mi::num_cus();
+  pp.resident = resident_groups(cus, head_dim);
+  pp.cus = head_dim == 256 ? 0 : cus;
+  const UnitLayout L = unit_layout(pp.resident, workspace_bytes, num_kv_heads, head_dim);
   static std::atomic<uint64_t> plans{0};
   pp.serial = (plans.fetch_add(1, std::memory_order_relaxed) + 1) * 0x9e3779b97f4a7c15ull;
   pp.key = run_key(workspace, workspace_bytes, num_kv_heads, pp.group, head_dim, static_cast<hipStream_t>(stream));
@@ -1353,17 +1367,21 @@ extern "C" int mi_prefill_run(void* workspace, size_t workspace_bytes, const voi
     return mi::fail(MI_ERR_INVALID, "prefill run: q rows, out rows and pool must be 16-byte aligned");
   if (q_stride_token < 0 || q_stride_head < 0 || out_stride_token < 0 || out_stride_head < 0)
     return mi::fail(MI_ERR_INVALID, "prefill run: negative stride");
-  const int64_t grid = run_groups(batch_size, total_q, num_qo_heads / num_kv_heads, num_kv_heads, head_dim);
+  const int resident = resident_groups(mi::num_cus(), head_dim);
+  const int64_t grid = run_groups(resident, batch_size, total_q, num_qo_heads / num_kv_heads, num_kv_heads, head_dim);
   if (grid > 0x7fffffff) return mi::fail(MI_ERR_INVALID, "prefill run: too many tiles");
   char* ws = static_cast<char*>(workspace);
   RunParams rp;
   rp.header = reinterpret_cast<const PrefillHeader*>(ws);
   rp.tiles = reinterpret_cast<const PrefillTile*>(ws + 256);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const UnitLayout L = unit_layout(workspace_bytes, num_kv_heads, head_dim);
+  const UnitLayout L = unit_layout(resident, workspace_bytes, num_kv_heads, head_dim);
   rp.unit_serial = reinterpret_cast<const uint64_t*>(ws + L.off);
   rp.units = reinterpret_cast<const PrefillTile*>(ws + L.off + 256);
   rp.parts = ws + L.parts;
+  rp.last_tile = int(std::min<size_t>(tile_capacity(batch_size, total_q), 1 << 30)) - 1;
+  rp.last_unit = std::max(L.capacity, 1) - 1;
+  rp.max_units = int(grid / num_kv_heads);
   rp.key = run_key(workspace, workspace_bytes, num_kv_heads, num_qo_heads / num_kv_heads, head_dim, s);
   rp.q = static_cast<const uint16_t*>(q);
   rp.q_st = q_stride_token;
