@@ -216,7 +216,8 @@ typedef void (*LinearKernel)(LinearParams);
 // are then no more than W.  With up to one tile per CU the loads in flight of a
 // workgroup bound it (D 4, as for long K); two tiles when the launch is so long
 // that starting and ending workgroups shows.  With two blocks of x, what bounds
-// it is x from L2, so as many tiles as still leave workgroups for the CUs.
+// it is x from L2, so as many tiles as still leave workgroups for the CUs (512 tiles
+// in fours leave half of them idle: 8,192 x 7,168, 32 rows, 29.5 us, library 25.7).
 // Half tiles up to 128 tiles (full ones leave half of the CUs or more idle), with
 // two blocks of x, which they read twice as often, for long k only (us at 8 / 32 rows,
 // whole / half): 896 x 4,864 6.8 / 10.3, 5.6 / 9.2; 2,048 x 8,960 11.4 / 18.1, 9.1 / 15.7;
@@ -230,11 +231,11 @@ LinearKernel pick_kernel(int tiles, int k, int mb, int* cols) {
     *cols = 8;
     return pick<1, 4, false, true>(mb);
   }
-  const int r = mb == 1 ? (tiles > 2048 ? 2 : 1) : tiles <= 256 ? 1 : tiles < 512 ? 2 : 4;
+  const int r = mb == 1 ? (tiles > 2048 ? 2 : 1) : tiles <= 256 ? 1 : tiles <= 512 ? 2 : 4;
   *cols = 16 * r;
   if (mb == 1 && (r == 2 || (tiles > 256 && k < 8192))) return r == 2 ? pick<2, 2>(1) : pick<1, 2>(1);
   if (mb == 1) return linear_kernel<1, 1, 4, false, false>;
-  return r == 1 ? pick<1, 2>(2) : r == 2 ? pick<2, 2>(2) : pick<4, 2>(2);
+  return r == 1 ? pick<1, 2>(2) : r == 2 ? pick<2, 2>(2) : linear_kernel<4, 2, 2, false, false>;
 }
 
 // With the gated product, from the pairs of a gate and an up tile (us at 8 / 32

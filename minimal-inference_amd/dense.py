@@ -85,13 +85,15 @@ LINEAR_MAX_K = 1 << 23
 
 
 def _few_rows(rows: int, n: int, k: int) -> bool:
-    """Whether the few-row kernel is the faster one: up to 16 rows everywhere but on
-    the largest weights of long rows (59,136 x 8,192, 16 rows: 181 us, library 170),
-    up to 32 while k is short (4,096 x 14,336: 34 us, library 31; 28,672 x 4,096:
-    46 us, library 55)."""
+    """Whether the few-row kernel is the faster one (us, kernel and library).  Up to 16
+    rows everywhere but on the largest weights of long rows (59,136 x 8,192, 16 rows:
+    181, 170) and those of a few more tiles than it has workgroups at once (10,240 x
+    8,192, 16 rows: 38.2, 34.5; 8 rows 35.9, 34.3); up to 32 while k is short (4,096 x
+    14,336: 34, 31; 28,672 x 4,096: 46, 55), from 5,120 on without the weights of a
+    little over one round of four tiles each (18,432 x 5,120: 46, 43)."""
     if rows <= 16:
-        return k < 8192 or n <= 32768
-    return rows <= LINEAR_MAX_ROWS and k < 8192
+        return k < 8192 or n <= 8192 or 16384 <= n <= 32768
+    return rows <= LINEAR_MAX_ROWS and (k < 5120 or (k < 8192 and not 16384 < n <= 32768))
 
 
 def _plain(*tensors: torch.Tensor | None) -> bool:
@@ -138,7 +140,9 @@ def linear_silu(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor:
     runs on the few-row kernel."""
     rows, k = x.shape
     n = gate_up.shape[0] // 2
-    if n % 16 or gate_up.shape[0] % 2 or not _takes(x, gate_up, None):
+    # (over 16 long rows the pairs of tiles hold too many registers: 51,200 x 5,120, 32
+    # rows, 113 us, library and SiLU kernel 96)
+    if n % 16 or gate_up.shape[0] % 2 or (rows > 16 and k >= 5120) or not _takes(x, gate_up, None):
         return silu_mul(linear(x, gate_up))
     out = torch.empty(rows, n, dtype=x.dtype, device=x.device)
     _lib.call("mi_linear_silu", x.data_ptr(), x.stride(0), gate_up.data_ptr(), out.data_ptr(), n, rows, n, k,
