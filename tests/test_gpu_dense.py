@@ -137,9 +137,11 @@ def test_few_row_linear(dev, rows, n, k):
     bf16 values; x rows and out rows strided, and the columns and rows around
     them untouched.
 
-    Bound: the sum of k products in fp32, in any order, is within
-    k * 2^-24 * sum |x w| of the exact one, and the result is rounded once to
-    bf16 (2^-8 relative); the reference's own fp32 error is of the first kind."""
+    Bound: rounding errors of a sum of k products in fp32 are independent enough to
+    stay within 4 sqrt(k) 2^-24 sum |x w| of the exact one (the worst case, k in the
+    place of 4 sqrt(k), is 27 at k = 18,944 and would hide a lost slab of 64 k, 8),
+    and the result is rounded once to bf16 (2^-8 relative); the reference's own fp32
+    error is of the first kind."""
     from minimal_inference_amd import _lib
 
     g = torch.Generator(device=dev).manual_seed(rows * 131 + n + k)
@@ -154,12 +156,32 @@ def test_few_row_linear(dev, rows, n, k):
         ref = x.float() @ w.float().t() + b
         mag = x.float().abs() @ w.float().abs().t() + (0.0 if bias is None else bias.float().abs())
         err = (out[:rows, :n].float() - ref).abs()
-        assert bool((err <= 2 ** -8 * ref.abs() + 2 * k * 2 ** -24 * mag).all())
+        assert bool((err <= 2 ** -8 * ref.abs() + 2 * 4 * k ** 0.5 * 2 ** -24 * mag).all())
         assert bool((out[rows] == 7.0).all()) and bool((out[:, n:] == 7.0).all())
         again = torch.empty_like(out)
         _lib.call("mi_linear", x.data_ptr(), x.stride(0), w.data_ptr(), bias.data_ptr() if bias is not None else None,
                   again.data_ptr(), again.stride(0), rows, n, k, torch.cuda.current_stream().cuda_stream)
         assert torch.equal(again[:rows, :n], out[:rows, :n])
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 32])
+@pytest.mark.parametrize("n,k", [
+    (16, 64), (48, 192), (896, 4864), (4096, 320), (4112, 4096), (8192, 576), (8208, 576), (32768, 256), (32784, 320),
+    (512, 8192), (16, 18944), (16, 18880), (2048, 1984), (2048, 2112), (4608, 9024),
+])
+def test_few_row_linear_of_whole_numbers(dev, rows, n, k):
+    """Whole numbers up to 8: every sum is exact in fp32 in any order, so the result
+    is the exact one's bf16, and a part of k that is lost or taken twice moves it."""
+    from minimal_inference_amd import _lib
+
+    g = torch.Generator(device=dev).manual_seed(rows * 131 + n + k)
+    x = torch.randint(-8, 9, (rows, k), device=dev, generator=g).to(torch.bfloat16)
+    w = torch.randint(-8, 9, (n, k), device=dev, generator=g).to(torch.bfloat16)
+    out = torch.empty(rows, n, device=dev, dtype=torch.bfloat16)
+    _lib.call("mi_linear", x.data_ptr(), k, w.data_ptr(), None, out.data_ptr(), n, rows, n, k,
+              torch.cuda.current_stream().cuda_stream)
+    assert 64 * k < 2 ** 24
+    assert torch.equal(out, (x.float() @ w.float().t()).to(torch.bfloat16))
 
 
 def test_few_row_linear_routes(dev):
