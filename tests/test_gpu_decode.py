@@ -397,3 +397,41 @@ def test_splits_merged_in_two_levels(dev, parity, hq, hkv, d, ctx, nsplit):
     outs = [w.run(q, pool).cpu() for _ in range(3)]
     parity(outs[0].float(), _ref(b))
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("hq,hkv,d,ctx", [(32, 8, 128, 16 * 97 + 5), (28, 4, 128, 16 * 120), (14, 2, 64, 16 * 260), (16, 4, 256, 16 * 65)])
+def test_infinities_and_nan_in_two_level_merges(dev, parity, hq, hkv, d, ctx):
+    """Values that no level of the merge may lose or spread: V infinite or NaN for
+    one key, whole splits and groups whose scores are all -inf, K infinite for one
+    key (its request's rows are NaN)."""
+    b = make_paged_batch([17, ctx, 200], hq, hkv, d, seed=ctx + d)
+    b["q"][..., 0] = 1.0
+    first, group = b["indptr"][1], hq // hkv
+    w = _wrapper(dev)
+    _, q, ip, ix, lp = to_dev(b, dev)
+    w.plan(ip, ix, lp, hq, hkv, d, 16)
+    items = w._ws[256:256 + 128 * 600].view(torch.int32).view(-1, 32).cpu()
+    of_request = items[(items[:, 24] == 1) & (items[:, 29] > 0) & (items[:, 29] < 1 << 16)]
+    assert int(of_request[0, 29]) > (36 if d == 64 else 16 if group * d > 512 else 24)
+
+    def run(pool):
+        return w.run(q, pool.to(dev)).float().cpu()
+
+    clean = run(b["pool"])
+    page = int(b["indices"][first + 50])
+    pool = b["pool"].clone()
+    pool[page, 1, 7, 0, 3] = float("inf")
+    pool[page, 1, 7, hkv - 1, 5] = float("nan")
+    out = run(pool)
+    assert bool(torch.isposinf(out[1, :group, 3]).all()) and bool(out[1, hq - group:, 5].isnan().all())
+    out[1, :group, 3], out[1, hq - group:, 5] = clean[1, :group, 3], clean[1, hq - group:, 5]
+    assert torch.equal(out, clean)
+    pages = (ctx + 15) // 16
+    hidden = b["indices"][first + 3:first + pages * 3 // 4].long()
+    pool = b["pool"].clone()
+    pool[hidden, 0, :, :, 0] = float("-inf")
+    parity(run(pool), _ref({**b, "pool": pool}))
+    pool = b["pool"].clone()
+    pool[page, 0, 7, :, 0] = float("inf")
+    out = run(pool)
+    assert bool(out[1].isnan().all()) and torch.equal(out[::2], clean[::2])

@@ -234,20 +234,23 @@ def test_long_prompt_4096(dev, parity):
     parity(out, ref)
 
 
-# (heads, new rows per request, cached tokens per request, row blocks per wave the plan picks)
+# (heads, new rows per request, cached tokens per request, row blocks per wave the
+# plan picks, KV tiles per unit at most, units)
 SPLIT_CASES = [
-    ((32, 8, 128), [3], [1000], 1),             # one short tile per KV head, cut at kMinChunk
-    ((28, 4, 128), [193, 1, 64], [900, 65, 0], 1),  # fine tiles, ragged, one that is not split
-    ((8, 1, 64), [2], [9000], 1),               # a single tile: the most units one merge takes
-    ((64, 8, 128), [200, 37], [5001, 3000], 3),  # coarse tiles of three row blocks
-    ((14, 2, 64), [700], [4010], 2),
-    ((16, 4, 256), [70], [2500], 1),
+    ((32, 8, 128), [3], [1000], 1, 4, 4),             # one short tile per KV head, cut at kMinChunk
+    ((28, 4, 128), [193, 1, 64], [900, 65, 0], 1, 4, 106),  # fine tiles, ragged, some that are not split
+    ((8, 1, 64), [2], [9000], 1, 8, 18),              # a single tile of 141 KV tiles, cut at sqrt(141 / 2)
+    ((64, 8, 128), [200, 37], [5001, 3000], 3, 14, 62),  # coarse tiles of three row blocks
+    ((14, 2, 64), [700], [4010], 2, 8, 353),
+    ((16, 4, 256), [70], [2500], 1, 4, 52),
+    # more tiles than the plan's block has threads, over two resident rounds, the last one split
+    ((8, 1, 64), [144] * 60 + [8], [0] * 60 + [9000], 1, 8, 1098),
 ]
 
 
-@pytest.mark.parametrize("heads,qo_lens,cached,blocks", SPLIT_CASES)
+@pytest.mark.parametrize("heads,qo_lens,cached,blocks,chunk,units", SPLIT_CASES)
 @pytest.mark.parametrize("causal", [True, False])
-def test_tiles_split_over_the_keys(dev, parity, heads, qo_lens, cached, blocks, causal):
+def test_tiles_split_over_the_keys(dev, parity, heads, qo_lens, cached, blocks, chunk, units, causal):
     """Tiles cut into units along the keys: against the oracle, the same bits
     on every run of a plan (the merge counters are back at zero), and with a
     workspace that has no room for partials (nothing is split)."""
@@ -274,7 +277,7 @@ def test_tiles_split_over_the_keys(dev, parity, heads, qo_lens, cached, blocks, 
         return ws[:32].view(torch.int32).tolist(), outs
 
     header, outs = run(128 << 20)
-    assert header[1] == 0 and header[3] == blocks and header[4] > 0  # no error, the form, a split
+    assert header[1] == 0 and header[3] == blocks and header[4] == chunk and header[6] == units
     parity(outs[0].float(), ref)
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
     header, whole = run(int(_lib.load().mi_prefill_workspace_size(len(qo_lens), total)))
@@ -397,3 +400,121 @@ def test_saved_plans_and_other_geometry_take_whole_tiles(dev, heads, qo_lens, ca
     flipped, _ = c.plan(c.need)
     assert torch.equal(out2[:, hq:], flipped.run(c.q[1], pool2[:, :, :, hkv:].contiguous()))
     assert torch.equal(c.ws, kept)
+
+
+def test_few_partial_slots_bind_the_split(dev, parity):
+    """A workspace with room for two slots of coarse units (five of fine ones): two
+    tiles of 32 KV tiles that are cut into eight units each where there is room are
+    cut into two, and merged from them."""
+    c = _Planned(dev, (32, 8, 128), [20], [2000], seed=34)
+    assert c.ws[16:28].view(torch.int32).tolist()[::2] == [4, 16]  # chunk, units
+    w, ws = c.plan(2300 << 10)
+    assert ws[16:28].view(torch.int32).tolist()[::2] == [16, 4]
+    outs = [w.run(c.q[0], c.pool) for _ in range(3)]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert not torch.equal(outs[0], c.whole[0])
+    parity(outs[0].float().cpu(), c.whole[0].float().cpu())
+
+
+def test_more_requests_than_the_plans_threads(dev, parity):
+    """1,100 requests of 1 to 40 rows, some of none, some on cached tokens."""
+    g = torch.Generator().manual_seed(35)
+    qo_lens = torch.randint(0, 41, (1100,), generator=g).tolist()
+    kv_lens = [n + (100 if i % 7 == 0 else 0) for i, n in enumerate(qo_lens)]
+    b = make_paged_batch(kv_lens, 4, 2, 64, seed=35)
+    out, ref = _run(dev, b, qo_lens, 4, 2, 64, seed=35)
+    parity(out, ref)
+
+
+@pytest.mark.parametrize("heads,qo_lens,cached", OWNED_CASES)
+def test_split_tiles_with_head_major_rows(dev, heads, qo_lens, cached):
+    """q and out with other strides on split tiles of every form: head-major, and
+    rows further apart than their heads; the bits of contiguous ones, nothing
+    written between the rows."""
+    c = _Planned(dev, heads, qo_lens, cached, seed=36)
+    hq, _, d = heads
+    q = c.q[0].transpose(0, 1).contiguous().transpose(0, 1)
+    out = torch.full((hq, c.total, d), float("nan"), dtype=torch.bfloat16, device=dev).transpose(0, 1)
+    c.w.run(q, c.pool, out=out)
+    assert torch.equal(out, c.units[0])
+    wide = torch.full((c.total, hq + 3, d + 8), 7.0, dtype=torch.bfloat16, device=dev)
+    wide_q = wide.clone()
+    wide_q[:, 1:1 + hq, :d] = c.q[0]
+    c.w.run(wide_q[:, 1:1 + hq, :d], c.pool, out=wide[:, 2:2 + hq, :d])
+    assert torch.equal(wide[:, 2:2 + hq, :d], c.units[0])
+    wide[:, 2:2 + hq, :d] = 7.0
+    assert bool((wide == 7.0).all())
+
+
+def test_plans_with_and_without_units_under_one_graph(dev):
+    """Plans in turn that split and do not, in one workspace, each followed by an
+    eager run and a replay of the run captured under the first."""
+    split = _Planned(dev, (32, 8, 128), [40, 3], [2000, 1000], seed=37)
+    flat = _Planned(dev, (32, 8, 128), [20, 23], [0, 30], seed=38)
+    split.plan(0, ws=split.ws)
+    q, pool = split.q[0].clone(), torch.zeros(max(split.pool.shape[0], flat.pool.shape[0]), *split.pool.shape[1:],
+                                              dtype=torch.bfloat16, device=dev)
+    indices = torch.zeros(max(split.csr[2].numel(), flat.csr[2].numel()), dtype=torch.int32, device=dev)
+    static = [t.clone() for t in split.csr[:2]] + [indices, split.csr[3].clone()]
+    w = split.w
+    w.plan(*static, 32, 8, 128, 16, causal=True, max_total_q=split.total)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = w.run(q, pool)
+    for c in (split, flat, split, split, flat, flat, split):
+        for t, v in zip(static, c.csr):
+            t[:v.numel()].copy_(v)
+        pool[:c.pool.shape[0]].copy_(c.pool)
+        w.plan(*static, 32, 8, 128, 16, causal=True, max_total_q=c.total)
+        assert (int(w._ws[16:20].view(torch.int32)[0]) > 0) == (c is split)
+        for k in range(2):
+            q.copy_(c.q[k])
+            graph.replay()
+            assert torch.equal(captured, c.whole[k])
+            assert torch.equal(w.run(q, pool), c.units[k])
+
+
+@pytest.mark.parametrize("heads,qo_lens,cached", OWNED_CASES)
+def test_infinities_and_nan_in_split_tiles(dev, heads, qo_lens, cached):
+    """Values that no merge may lose or spread: V infinite or NaN for one key, a
+    run of keys (several units' worth) whose scores are all -inf, K infinite for
+    one key (a row that sees it is NaN)."""
+    c = _Planned(dev, heads, qo_lens, cached, seed=39)
+    hq, hkv, d = heads
+    group, ip, ix = hq // hkv, c.csr[1].tolist(), c.csr[2].long()
+    q = c.q[0].clone()
+    q[..., 0] = 1.0
+
+    def page(token):  # of the first request
+        return int(ix[ip[0] + token // 16]), token % 16
+
+    far = cached[0] - 70
+    clean = c.w.run(q, c.pool).float()
+    pool = c.pool.clone()
+    pg, row = page(far)
+    pool[pg, 1, row, 0, 3] = float("inf")
+    pool[pg, 1, row, hkv - 1, 5] = float("nan")
+    out = c.w.run(q, pool).float()
+    n0 = qo_lens[0]
+    assert bool(torch.isposinf(out[:n0, :group, 3]).all())
+    assert bool(out[:n0, hq - group:, 5].isnan().all())
+    out[:n0, :group, 3] = clean[:n0, :group, 3]
+    out[:n0, hq - group:, 5] = clean[:n0, hq - group:, 5]
+    assert torch.equal(out, clean)
+    # the first 3/4 of the cached pages out of sight
+    pool = c.pool.clone()
+    hidden = ix[ip[0]:ip[0] + cached[0] // 16 * 3 // 4]
+    pool[hidden, 0, :, :, 0] = float("-inf")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        whole = c.w.run(q, pool)
+    side.synchronize()
+    out = c.w.run(q, pool)
+    assert bool(out.isfinite().all()) and not torch.equal(out[:n0].float(), clean[:n0])
+    # (two correct results: P is rounded to bf16 against other maxima, 2^-8 each)
+    assert bool(((out.float() - whole.float()).abs() <= 2 ** -6 * whole.float().abs().clamp(min=1.0)).all())
+    pool = c.pool.clone()
+    pool[pg, 0, row, :, 0] = float("inf")
+    out = c.w.run(q, pool)
+    assert bool(out[:n0].isnan().all()) and torch.equal(out[n0:].float(), clean[n0:])
