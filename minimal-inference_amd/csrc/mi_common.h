@@ -35,9 +35,6 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return uint16_t(u >> 16);
 }
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return uint32_t(f32_to_bf16(lo)) | (uint32_t(f32_to_bf16(hi)) << 16);
-}
 // The same rounding (to nearest even) in one gfx950 instruction
 // (v_cvt_pk_bf16_f32) per pair, for kernel outputs: finite values convert
 // bit-identically to f32_to_bf16; a NaN comes out as a quiet NaN.

@@ -58,21 +58,11 @@ constexpr int kPageSize = 16;
 constexpr int kMinRows = 8;    // fewest query positions per workgroup (head_dim 256, group 8)
 constexpr int kKvTile = 64;    // keys per staged tile (4 pages)
 constexpr float kLazyRescale = 8.0f;
-// 32-byte row pad: the transpose reads of V (four rows x 32 bytes per
-// 16 lanes) and the 16-byte K reads both land on distinct banks (a 16-byte
-// pad measured 13.9M bank-conflict cycles per launch on the Mistral-7B
-// batch, 32 bytes none).
-#ifndef PREFILL_RS_PAD
-#define PREFILL_RS_PAD 32
-#endif
 // K / V tiles staged straight to LDS by the gfx950 buffer loads with the
 // `lds` modifier (no staging registers, no LDS store instructions).  A wave's
 // load instruction fills 1 KB of LDS, lane l at byte 16 l, so the rows are
 // unpadded and a 16-byte chunk's place in its row is permuted instead
 // (chunk_slot) to keep the reads off shared banks.
-#ifndef PREFILL_DMA
-#define PREFILL_DMA 1
-#endif
 // Output staging: pad bytes after every 8 columns (32 bytes each) of a
 // column-major 16-row block, so the 8-byte writes of a half wave and the
 // transpose reads of two lane groups fall on distinct banks.
@@ -614,7 +604,6 @@ typedef __attribute__((address_space(3))) char lds_t;
 
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2_t;
 
-__device__ __forceinline__ void lds_store16(lds_t* p, u32x4_t v) { *(__attribute__((address_space(3))) u32x4_t*)p = v; }
 __device__ __forceinline__ void lds_store8(lds_t* p, u32x2_t v) { *(__attribute__((address_space(3))) u32x2_t*)p = v; }
 __device__ __forceinline__ u32x4_t lds_load16(const lds_t* p) {
   return *(const __attribute__((address_space(3))) u32x4_t*)p;
@@ -658,7 +647,7 @@ __device__ __forceinline__ float sum_xor32(float x) {
 // the rows are unpadded: c XOR a per-row value.  Measured with
 // SQ_LDS_BANK_CONFLICT on the Mistral-7B / Qwen2.5-72B head batches (per
 // launch): no permutation 70.8M / 210.8M conflict cycles; XOR (r & 15) 6.8M /
-// 16.8M; XOR 2 (r & 7) 1.8M / 1.9M (what the 32-byte row pad gave), so the 8
+// 16.8M; XOR 2 (r & 7) 1.8M / 1.9M (what rows padded by 32 bytes gave), so the 8
 // rows of a K read group and the 4 rows x 32 bytes of a V transpose-read
 // group land on distinct banks.  128-byte rows (head_dim 64) put two rows in
 // a bank period and take XOR 2 ((r >> 1) & 3).
@@ -677,7 +666,7 @@ struct PrefillTraits {
   static constexpr int CPR = D / 8;                // 16-byte chunks per token row
   static constexpr int LOADS = kKvTile * CPR / THREADS;  // 16-byte loads per thread per tile, K and V each
   static_assert(LOADS >= 1 && kKvTile * CPR % THREADS == 0, "tile staging split");
-  static constexpr int RS = PREFILL_DMA ? D * 2 : D * 2 + PREFILL_RS_PAD;  // LDS row stride
+  static constexpr int RS = D * 2;                 // LDS row stride
   static constexpr int TILE = kKvTile * RS;        // bytes of one staged K or V tile
   static constexpr int MAXRB = MAXRB_;             // row blocks per wave
   static constexpr int OUT_BLK = 8 * 32 + kOutPad;  // output staging: bytes per 8 columns
@@ -892,9 +881,8 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
       unsigned(t.kt) >> 16 == kToEnd ? 0x7fffffff : int(unsigned(t.kt) >> 16)));
   const int kt0 = t.kt & 0xffff;
 
-  // ---- staging.  Load i of a thread covers token ltok + TPL i of the tile
-  // and 16-byte chunk ldc of that token's row: a wave's 64 lanes cover whole
-  // rows of one page (1 KB <= 16 rows), so the page id is wave-uniform -- a
+  // ---- staging.  A load of a wave covers whole rows of one page (1 KB <= 16
+  // rows), so the page id is wave-uniform -- a
   // scalar load, fetched one tile ahead -- and each page gets a buffer
   // descriptor (size 0 past the request's pages; on the request's last page
   // the size stops after its valid V rows, so the V rows past kv_len read as
@@ -906,7 +894,6 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
   const int npages_req = (t.kv_len + kPageSize - 1) / kPageSize;
   const int last_rows = t.kv_len - (npages_req - 1) * kPageSize;
   int voff[T::LOADS], pit[T::LOADS];
-#if PREFILL_DMA
   // Load i of wave w fills 1 KB block b = WAVES i + w of the tile: RPB rows,
   // lane l taking row b RPB + l / CPR and slot l % CPR of it, i.e. the chunk
   // chunk_slot(row, slot) (the permutation is its own inverse); a block lies
@@ -919,17 +906,6 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
     pit[i] = __builtin_amdgcn_readfirstlane(bk * RPB / kPageSize);
     voff[i] = (tr % kPageSize) * tok_bytes + hkv * D * 2 + chunk_slot<D>(tr, lane % T::CPR) * 16;
   }
-#else
-  constexpr int TPL = T::THREADS / T::CPR;
-  const int ltok = int(threadIdx.x) / T::CPR, ldc = int(threadIdx.x) - ltok * T::CPR;
-#pragma unroll
-  for (int i = 0; i < T::LOADS; ++i) {
-    const int tt = ltok + TPL * i;
-    pit[i] = __builtin_amdgcn_readfirstlane(tt / kPageSize);
-    voff[i] = (tt % kPageSize) * tok_bytes + hkv * D * 2 + ldc * 16;
-  }
-  u32x4_t kreg[T::LOADS], vreg[T::LOADS];
-#endif
   int pid[T::LOADS];
   // page ids through the constant address space: a uniform index then
   // compiles to a scalar load (kv_indices is not written during the launch)
@@ -955,36 +931,15 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
       const int size = !ok ? 0 : (pg_idx == npages_req - 1 ? kv_bytes + last_rows * tok_bytes : page_bytes);
       const char* base = reinterpret_cast<const char*>(p.pool) + (ok ? int64_t(pg) * page_bytes : 0);
       const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, size, kBufferWord3);
-#if PREFILL_DMA
       lds_t* kdst = lds + buf * 2 * T::TILE + 1024 * (T::WAVES * i + w);
       lds_dma16(rs, kdst, voff[i], 0);
       lds_dma16(rs, kdst + T::TILE, voff[i], kv_bytes);
-#else
-      (void)buf;
-      kreg[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[i], 0, 0);
-      vreg[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, voff[i], kv_bytes, 0);
-#endif
     }
   };
-  auto store_tile = [&](int buf) {
-#if !PREFILL_DMA
-    lds_t* kl = lds + buf * 2 * T::TILE + ltok * T::RS + ldc * 16;
-    lds_t* vl = kl + T::TILE;
-#pragma unroll
-    for (int i = 0; i < T::LOADS; ++i) {
-      lds_store16(kl + TPL * i * T::RS, kreg[i]);
-      lds_store16(vl + TPL * i * T::RS, vreg[i]);
-    }
-#else
-    (void)buf;
-#endif
-  };
-
   if (kt0 < ntile) {
     fetch_ids(kt0);
     load_tile(kt0, 0);
     fetch_ids(kt0 + 1);
-    store_tile(0);
   }
   // Everything loaded so far (Q, tile 0, the next page ids) is waited for
   // here, so the loop head carries no pending load from before the loop;
@@ -1000,12 +955,11 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
   int koff[T::KSTEPS], voff_lds[T::NT];
 #pragma unroll
   for (int s2 = 0; s2 < T::KSTEPS; ++s2)
-    koff[s2] = PREFILL_DMA ? n * T::RS + chunk_slot<D>(n, 4 * s2 + g) * 16 : n * T::RS + (4 * s2 + g) * 16;
+    koff[s2] = n * T::RS + chunk_slot<D>(n, 4 * s2 + g) * 16;
 #pragma unroll
   for (int j = 0; j < T::NT; ++j) {
     const int vr = 4 * g + (n >> 2);
-    voff_lds[j] = PREFILL_DMA ? vr * T::RS + chunk_slot<D>(vr, 2 * j + ((n & 3) >> 1)) * 16 + (n & 1) * 8
-                              : vr * T::RS + (n & 3) * 8 + 32 * j;
+    voff_lds[j] = vr * T::RS + chunk_slot<D>(vr, 2 * j + ((n & 3) >> 1)) * 16 + (n & 1) * 8;
   }
 
   for (int kt = kt0; kt < ntile; ++kt) {
@@ -1130,7 +1084,6 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
           }
           // ---- O += P V over key blocks (2h, 2h + 1)
           const lds_t* v0 = vl + 2 * h * 16 * T::RS;
-#if PREFILL_DMA
           // The transpose reads go through inline asm here: with the builtin the
           // compiler waited for every load to LDS in flight (the next tile's)
           // before the first of them.  One statement per group of 4 columns:
@@ -1165,25 +1118,11 @@ __device__ __forceinline__ void run_unit(const RunParams& p, const PrefillTile& 
               for (int r = 0; r < T::MAXRB; ++r) o[r][j0 + jj] = mi::mfma_16x16x32_bf16(pa[r], vb, o[r][j0 + jj]);
             }
           }
-#else
-          const lds_t* v1 = v0 + 16 * T::RS;
-#pragma unroll
-          for (int j = 0; j < T::NT; ++j) {
-            const s16x4_t a = lds_read_tr16(v0 + voff_lds[j]), b = lds_read_tr16(v1 + voff_lds[j]);
-            const mi::bf16x8_t vb =
-                __builtin_bit_cast(mi::bf16x8_t, (s16x8_t){a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
-#pragma unroll
-            for (int r = 0; r < T::MAXRB; ++r) o[r][j] = mi::mfma_16x16x32_bf16(pa[r], vb, o[r][j]);
-          }
-#endif
         }
       }
     }
-    if (kt + 1 < ntile) store_tile(buf ^ 1);
-#if PREFILL_DMA
     // the next tile's rows are in LDS (the loads went straight there)
     if (kt + 1 < ntile) __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-#endif
     __syncthreads();
   }
 
