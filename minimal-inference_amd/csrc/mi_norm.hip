@@ -121,13 +121,16 @@ struct SiluMulParams {
 // division per thread it was VALU bound: 18,240 x 14,336 295-318 us = 4.9 TB/s, now
 // 251-272 us = 5.8 TB/s; 8,000 x 29,568 277 -> 234 us; 2,000 x 14,336 35 -> 30 us.
 // (1,024 or 4,096 workgroup rows that walk further cost 17 % and 9 %; the reciprocal
-// without its two steps gains 4 %.)
+// without its two steps gains 4 %; with the workgroup's shape read at run time the
+// whole workgroups of wide rows took 1 % longer: NARROW.)
 constexpr int kSiluThreads = 256;
+template <bool NARROW>
 __global__ __launch_bounds__(kSiluThreads) void silu_mul_kernel(SiluMulParams p) {
-  const int ch = int(blockIdx.x * blockDim.x + threadIdx.x);
+  const int bx = NARROW ? int(blockDim.x) : kSiluThreads, by = NARROW ? int(blockDim.y) : 1;
+  const int ch = int(blockIdx.x) * bx + int(threadIdx.x);
   if (ch * 8 >= p.inter) return;
-  const int64_t step = int64_t(gridDim.y) * blockDim.y;
-  for (int64_t row = int64_t(blockIdx.y) * blockDim.y + threadIdx.y; row < p.rows; row += step) {
+  const int64_t step = int64_t(gridDim.y) * by;
+  for (int64_t row = int64_t(blockIdx.y) * by + (NARROW ? threadIdx.y : 0); row < p.rows; row += step) {
     const uint16_t* g = p.gu + row * p.gu_stride + ch * 8;
     const uint4 gv = mi::load16_nt(g), uv = mi::load16_nt(g + p.inter);
     const uint32_t gw[4] = {gv.x, gv.y, gv.z, gv.w}, uw[4] = {uv.x, uv.y, uv.z, uv.w};
@@ -202,6 +205,6 @@ extern "C" int mi_silu_mul(const void* gate_up, int64_t gate_up_stride, void* ou
   const int chunks = intermediate / 8, parts = (chunks + kSiluThreads - 1) / kSiluThreads;
   const int bx = parts > 2 ? kSiluThreads : (chunks + parts - 1) / parts, by = kSiluThreads / bx;
   const dim3 grid(parts, uint32_t(std::min<int64_t>((rows + by - 1) / by, 65535)));
-  hipLaunchKernelGGL(silu_mul_kernel, grid, dim3(bx, by), 0, static_cast<hipStream_t>(stream), p);
+  hipLaunchKernelGGL(bx == kSiluThreads ? silu_mul_kernel<false> : silu_mul_kernel<true>, grid, dim3(bx, by), 0, static_cast<hipStream_t>(stream), p);
   return mi::check_launch("silu_mul_kernel");
 }
