@@ -474,6 +474,26 @@ def test_plans_with_and_without_units_under_one_graph(dev):
             assert torch.equal(w.run(q, pool), c.units[k])
 
 
+def test_plan_and_run_captured_together(dev):
+    """A captured plan lists whole tiles only, on every replay and for the eager runs
+    after it, whatever an eager plan left in the workspace."""
+    split = _Planned(dev, (32, 8, 128), [40, 3], [2000, 1000], seed=37)
+    static, q = [t.clone() for t in split.csr], split.q[0].clone()
+    w = split.w
+    w.plan(*static, 32, 8, 128, 16, causal=True, max_total_q=split.total)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        w.plan(*static, 32, 8, 128, 16, causal=True, max_total_q=split.total)
+        captured = w.run(q, split.pool)
+    for k in range(3):
+        q.copy_(split.q[k])
+        graph.replay()
+        assert torch.equal(captured, split.whole[k])
+        assert torch.equal(w.run(q, split.pool), split.whole[k])
+        w.plan(*static, 32, 8, 128, 16, causal=True, max_total_q=split.total)
+        assert torch.equal(w.run(q, split.pool), split.units[k])
+
+
 @pytest.mark.parametrize("heads,qo_lens,cached", OWNED_CASES)
 def test_infinities_and_nan_in_split_tiles(dev, heads, qo_lens, cached):
     """Values that no merge may lose or spread: V infinite or NaN for one key, a
