@@ -313,9 +313,11 @@ __device__ __forceinline__ void write_header(const PlanParams& p, int ntiles, in
 // Batches of more requests than the block has threads: one request per thread
 // and round, its place found by counting the requests ordered before it in
 // global memory; tiles only.
-__device__ void plan_large(const PlanParams& p, int* wsum) {
+__device__ void plan_large(const PlanParams& p, int* wsum, int* s_fit) {
   const int t = threadIdx.x, bm = p.bm[1];
   int total = 0;
+  if (t == 0) *s_fit = 0;
+  __syncthreads();
   for (int base = 0; base < p.batch; base += blockDim.x) {
     const int b = base + t;
     int nt = 0, start = 0;
@@ -326,15 +328,18 @@ __device__ void plan_large(const PlanParams& p, int* wsum) {
         const int qc = max(0, p.qo_indptr[c + 1] - p.qo_indptr[c]);
         if (qc > qo || (qc == qo && c < b)) start += (qc + bm - 1) / bm;
       }
-      if (start + nt <= p.capacity)
+      if (start + nt <= p.capacity) {
         for (int k = 0; k < nt; ++k)
           p.tiles[start + k] = make_tile(bm, qo, request_kv(p, b), p.qo_indptr[b], p.kv_indptr[b], nt, k);
+        atomicMax(s_fit, start + nt);
+      }
     }
     int chunk_total = 0;
     block_scan(nt, wsum, &chunk_total);
     total += chunk_total;
   }
-  if (t == 0) write_header(p, total, min(total, p.capacity), 1, 0, 0);
+  __syncthreads();
+  if (t == 0) write_header(p, total, *s_fit, 1, 0, 0);  // (a record that nothing wrote is never run)
 }
 
 // Tile order: requests by decreasing prompt length (ties by index), each
@@ -366,7 +371,7 @@ __global__ __launch_bounds__(kPlanThreads) void prefill_plan_kernel(PlanParams p
   __shared__ float s_sums[4][kPlanThreads / 64];
   __shared__ unsigned short s_n[kSplitTiles];
   if (p.batch > kPlanThreads) {
-    plan_large(p, wsum);
+    plan_large(p, wsum, &s_fit);
     return;
   }
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;

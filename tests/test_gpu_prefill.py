@@ -426,6 +426,25 @@ def test_more_requests_than_the_plans_threads(dev, parity):
     parity(out, ref)
 
 
+@pytest.mark.parametrize("batch", [1100, 300])
+def test_a_list_too_short_for_the_rows_counts_whole_requests(dev, batch):
+    """A plan told of fewer rows than qo_indptr has reports the error, and counts
+    only tiles that it has written: those of the requests that fit."""
+    from minimal_inference_amd.prefill import BatchPrefillWithPagedKVCacheWrapper
+
+    qo = torch.arange(batch + 1, dtype=torch.int32, device=dev) * 40  # three tiles of 16 rows each
+    pages = torch.arange(batch + 1, dtype=torch.int32, device=dev) * 3
+    ws = torch.full((1 << 20,), 0x5a, dtype=torch.uint8, device=dev)
+    w = BatchPrefillWithPagedKVCacheWrapper(ws, "NHD")
+    w.plan(qo, pages, torch.zeros(3 * batch, dtype=torch.int32, device=dev),
+           torch.full((batch,), 8, dtype=torch.int32, device=dev), 8, 1, 64, 16, causal=True, max_total_q=104)
+    capacity = 104 // 8 + batch + 1
+    num_tiles, error = ws[:8].view(torch.int32).tolist()
+    assert error == 1 and num_tiles == capacity // 3 * 3 and capacity % 3
+    records = ws[256:256 + 32 * (num_tiles + 1)].view(torch.int32).view(-1, 8).cpu()
+    assert bool((records[:num_tiles, 2] == 40).all()) and int(records[num_tiles, 2]) != 40
+
+
 @pytest.mark.parametrize("heads,qo_lens,cached", OWNED_CASES)
 def test_split_tiles_with_head_major_rows(dev, heads, qo_lens, cached):
     """q and out with other strides on split tiles of every form: head-major, and
